@@ -19,9 +19,9 @@
 //    none of a tile skip its math; the q-tile order is reversed so the longest
 //    rows start first.
 // Kernels: prefill_b32_kernel streams K/V tiles into LDS by DMA (pages of a
-// multiple of 16 tokens, or contiguous K/V; see the section below);
+// multiple of 8 tokens, or contiguous K/V; see the section below);
 // prefill_f16_kernel stages tiles through registers and looks up every key
-// row on its own (any page size); prefill_f32_kernel is the exact-fp32
+// row on its own (the other page sizes); prefill_f32_kernel is the exact-fp32
 // contiguous op.
 //
 // prefill_f16_kernel: the next 64-key tile's rows are fetched from HBM into
@@ -68,20 +68,10 @@ struct TileRegs {
   u32x4 v[KPT];
 };
 
-__device__ __forceinline__ int64_t pick4(const int64_t (&v)[4], int g) {
-  return g == 0 ? v[0] : g == 1 ? v[1] : g == 2 ? v[2] : v[3];
-}
-
 // Fetches the K/V rows of the 64-key tile starting at k0 into registers.
-// Rows at or beyond kv_len (or not addressable) read as zero.
-//
-// ALIGNED (contiguous K/V, or pages of a multiple of 16 tokens): the 16 keys
-// of each quarter of the tile share one page, so the page lookup is one
-// uniform (scalar) block-table read per quarter and rows are plain offsets
-// from it. Scalar reads complete on their own counter, so the vector loads of
-// the tile are issued back to back and stay in flight while the current tile
-// is computed. Otherwise every row is looked up on its own.
-template <int D, bool ALIGNED>
+// Rows at or beyond kv_len (or not addressable) read as zero. Every row is
+// looked up on its own.
+template <int D>
 __device__ __forceinline__ void load_tile(TileRegs<D>& r, const AttnParams& p, const f16* kp,
                                           const f16* vp, int b, int hk, int k0, int kv_len,
                                           int tid) {
@@ -89,23 +79,9 @@ __device__ __forceinline__ void load_tile(TileRegs<D>& r, const AttnParams& p, c
   constexpr int KCH = TileRegs<D>::KCH;
   constexpr int KPT = TileRegs<D>::KPT;
   constexpr int RPP = kThreads / CPR;  // rows per pass of the K loader
-  int64_t goff[4];
-  if constexpr (ALIGNED) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int key = k0 + 16 * g;
-      goff[g] = key < kv_len ? p.kv.row_offset(b, hk, key) : -1;
-    }
-  }
   auto row_off = [&](int row) -> int64_t {
     const int j = k0 + row;
-    if (j >= kv_len) return -1;
-    if constexpr (ALIGNED) {
-      const int64_t base = pick4(goff, row >> 4);
-      return base < 0 ? -1 : base + (int64_t)(row & 15) * D;
-    } else {
-      return p.kv.row_offset(b, hk, j);
-    }
+    return j < kv_len ? p.kv.row_offset(b, hk, j) : -1;
   };
   const int col = tid % CPR;
 #pragma unroll
@@ -156,7 +132,7 @@ __device__ __forceinline__ void store_tile(const TileRegs<D>& r, f16* sK, f16* s
   }
 }
 
-template <int D, bool ALIGNED>
+template <int D>
 __global__ __launch_bounds__(kThreads) void prefill_f16_kernel(AttnParams p) {
   constexpr int KSTEPS = D / 16;  // k-steps of S^T
   constexpr int DBLK = D / 32;    // 32-row blocks of O^T
@@ -224,14 +200,14 @@ __global__ __launch_bounds__(kThreads) void prefill_f16_kernel(AttnParams p) {
   const float c = p.scale_log2;
 
   TileRegs<D> regs;
-  if (ntiles > 0) load_tile<D, ALIGNED>(regs, p, kp, vp, b, hk, 0, kv_len, tid);
+  if (ntiles > 0) load_tile<D>(regs, p, kp, vp, b, hk, 0, kv_len, tid);
 
   for (int t = 0; t < ntiles; ++t) {
     const int k0 = t * kBN;
     __syncthreads();
     store_tile<D>(regs, sK, sVt, tid);
     __syncthreads();
-    if (t + 1 < ntiles) load_tile<D, ALIGNED>(regs, p, kp, vp, b, hk, k0 + kBN, kv_len, tid);
+    if (t + 1 < ntiles) load_tile<D>(regs, p, kp, vp, b, hk, k0 + kBN, kv_len, tid);
     if (k0 >= wave_lim_max) continue;
 
     // S^T[key][row]: two 32-key blocks.
@@ -318,12 +294,12 @@ __global__ __launch_bounds__(kThreads) void prefill_f16_kernel(AttnParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Tile-DMA prefill kernel (pages of a multiple of 16 tokens, or contiguous
+// Tile-DMA prefill kernel (pages of a multiple of 8 tokens, or contiguous
 // K/V): prefill_b32_kernel (32-key tiles). Design:
 //
 //  * K and V tiles go from HBM straight into LDS with buffer_load ... lds
 //    (16 bytes per lane), no staging registers. Each wave moves one slab of
-//    the tile (16 or 8 keys), which lies in one page, through one buffer
+//    the tile (8 keys), which lies in one page, through one buffer
 //    resource whose size covers only the slab's valid rows: rows past seqlen
 //    land in LDS as zeros.
 //  * LDS holds two K and two V tiles (double buffer, one barrier per tile;
@@ -493,7 +469,7 @@ __device__ __forceinline__ half8 ld_vt(const char* buf, const int* voff, int s, 
 
 // With NW waves per workgroup and BN-key tiles, wave w moves the slab of
 // SLAB = BN / NW keys starting at k0 + SLAB * w (one page: pages hold a
-// multiple of 16 tokens).
+// multiple of SLAB tokens).
 template <int D, int NW, int BN>
 struct Slab {
   static constexpr int SLAB = BN / NW;                  // keys per wave and tile
@@ -1297,14 +1273,19 @@ hipError_t launch_prefill(const AttnParams& p, int D, int dtype, hipStream_t str
       hipLaunchKernelGGL(prefill_f32_kernel<64>, grid, dim3(64 * kF32Waves), 0, stream, p);
     return hipGetLastError();
   }
-  const bool aligned = p.kv.paged ? (p.kv.PS % 16) == 0 : p.kv.stride_tok == p.kv.D;
+  // The tile-DMA kernel moves slabs of 8 keys, each through one buffer
+  // resource, so a slab must lie in one page. Pages of 8, 24, 40, ... tokens
+  // go there too: at 5 ragged chunks of up to 777 rows, 32/8 heads, D = 64,
+  // 8-token pages, 44 us against 105 us for the register-staged kernel, which
+  // keeps the sizes whose slabs would cross pages.
+  const bool aligned = p.kv.paged ? (p.kv.PS % 8) == 0 : p.kv.stride_tok == p.kv.D;
   const int ntq = (p.M + kBM - 1) / kBM;
   if (!aligned) {
     const dim3 grid((unsigned)ntq, (unsigned)p.Hq, (unsigned)p.B);
     if (D == 128)
-      hipLaunchKernelGGL((prefill_f16_kernel<128, false>), grid, dim3(kThreads), 0, stream, p);
+      hipLaunchKernelGGL(prefill_f16_kernel<128>, grid, dim3(kThreads), 0, stream, p);
     else
-      hipLaunchKernelGGL((prefill_f16_kernel<64, false>), grid, dim3(kThreads), 0, stream, p);
+      hipLaunchKernelGGL(prefill_f16_kernel<64>, grid, dim3(kThreads), 0, stream, p);
     return hipGetLastError();
   }
   if (use_packed_rows(p)) {
