@@ -1063,7 +1063,235 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
 }
 
 // fp32 contiguous attention (the reference's CPU path accepts fp32,
-// flashattention_custom/ops.py:19-31), in fp32 arithmetic on the vector ALUs.
+// flashattention_custom/ops.py:19-31) on the fp32 matrix instruction
+// v_mfma_f32_32x32x2_f32, whose products and sums are fp32.
+//
+// A workgroup owns 32 query rows of one (sequence, q head). Its four waves
+// take the 32-key tiles round-robin, each with its own online softmax state
+// and its own K and V stage in LDS, so no wave waits for another until the
+// four states are merged at the end; the short rows of a causal sequence and
+// small batches still spread over the device (a 1000-row head is 32
+// workgroups). Per tile a wave issues D/2 + D/2 MFMAs of 64 cycles each and
+// about 100 VALU instructions, so the matrix cores bound it. K's stage is
+// refilled under the PV product and V's under the next QK^T product, which
+// hides the fetch without a second stage.
+//  * S^T = K Q^T: lane (key = lane % 32, half) reads 16 bytes of its key row,
+//    four dims for four MFMAs; the d order inside a step is the same for Q.
+//    16-byte chunks are XOR-swizzled per row, so 32 rows at one column hit
+//    all banks.
+//  * O^T = V^T P^T: accumulator register r of S^T holds key
+//    8 (r / 4) + 4 half + r % 4 of the lane's row, which is the B operand of
+//    the MFMA over that pair of keys; the A operand takes D/32 consecutive
+//    dims per lane (one LDS read for the D/32 MFMAs of a key pair), so
+//    output block i, register r is dim (D/32) (8 (r / 4) + 4 half + r % 4) + i.
+//  * Rounding: a score is four partial sums of D/4 products, and the PV sums
+//    of 16 keys start from zero and are added to the running O, so only the
+//    chain over 16-key sums grows with the key count (error against 64 bits
+//    at 1000 keys, D = 128: 1.6e-7; 1.75e-7 on the vector ALUs; 3.3e-7 with
+//    one chain each).
+constexpr int kF32MfmaWaves = 4;
+
+struct F32Grid {
+  int ntq;       // 32-row tiles per q head
+  int units;     // by_unit: (sequence, KV head) pairs per XCD; else all (sequence, q head)s
+  int group;     // by_unit: q heads per unit; else 1
+  int by_unit;   // XCD x runs units x, x + 8, ... (8 divides their number)
+};
+
+template <int D>
+__global__ __launch_bounds__(64 * kF32MfmaWaves, 2) void prefill_f32_mfma_kernel(AttnParams p, F32Grid g) {
+  constexpr int BN = 32;
+  constexpr int ROWB = 4 * D;          // bytes per key row
+  constexpr int CH = D / 4;            // 16-byte chunks per row
+  constexpr int RPI = 1024 / ROWB;     // rows per wave-wide DMA
+  constexpr int TILE = BN * ROWB;
+  constexpr int NDMA = BN / RPI;       // DMA instructions per tile of K (and of V)
+  constexpr int KS = D / 8;
+  constexpr int DB = D / 32;
+  constexpr int NW = kF32MfmaWaves;
+  typedef float floatv __attribute__((ext_vector_type(DB)));
+  __shared__ __attribute__((aligned(1024))) char smem[NW * 2 * TILE];
+  __shared__ float s_m[NW][32];
+  __shared__ float s_l[NW][32];
+
+  // Longest rows first. With the (sequence, KV head) pairs divisible over the
+  // XCDs, all tiles of the q heads that share K/V run on one XCD's L2.
+  int slot = blockIdx.x, bh, r;
+  if (g.by_unit) {
+    const int x = slot & 7;
+    slot >>= 3;
+    const int per = g.units * g.group;
+    r = slot / per;
+    const int w = slot - r * per;
+    const int unit = x + 8 * (w / g.group);
+    bh = unit * g.group + w % g.group;
+  } else {
+    r = slot / g.units;
+    bh = slot - r * g.units;
+  }
+  const int q0 = (g.ntq - 1 - r) * 32;
+  const int b = bh / p.Hq;
+  const int hq = bh - b * p.Hq;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31;
+  const int half_id = lane >> 5;
+  const int qrow = q0 + col;
+  const int hk = p.kv_head(hq);
+  const int kv_len = p.kv_len(b);
+  const int qo = p.q_off(b);
+  const int ko = p.k_off(b);
+  const int wg_lim = hk < 0 ? 0 : row_key_limit(kv_len, p.causal, qo, ko, min(q0 + 32, p.M) - 1);
+  const int min_lim = row_key_limit(kv_len, p.causal, qo, ko, q0);
+  const int lim = row_key_limit(kv_len, p.causal, qo, ko, qrow);
+  const int ntiles = (wg_lim + BN - 1) / BN;
+
+  const char* kp = reinterpret_cast<const char*>(p.k);
+  const char* vp = reinterpret_cast<const char*>(p.v);
+  const int64_t kv_base = hk < 0 ? 0 : 4 * p.kv.row_offset(b, hk, 0);
+  char* sk = smem + wave * 2 * TILE;
+  char* sv = sk + TILE;
+  const int drow = lane / CH, dch = lane % CH;
+  // rows past kv_len lie outside the buffer range and land as zeros; a tile
+  // past the last has an empty range (no memory access), so the loop has no
+  // branch around its DMAs
+  auto dma = [&](const char* base, int t, char* dst, bool swizzle) {
+    const int k0 = t * BN;
+    const int rows = t < ntiles ? min(BN, kv_len - k0) : 0;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        make_rsrc(base + kv_base + (int64_t)(rows > 0 ? k0 : 0) * ROWB, (uint32_t)(rows * ROWB));
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+      const int row = RPI * i + drow;
+      lds_dma16<false>(rsrc, dst + 1024 * i,
+                       (uint32_t)(row * ROWB + 16 * (swizzle ? dch ^ (row % CH) : dch)));
+    }
+  };
+  int t = wave;
+  dma(kp, t, sk, true);
+  dma(vp, t, sv, false);
+
+  const float* qp = reinterpret_cast<const float*>(p.q) +
+                    (((int64_t)b * p.Hq + hq) * p.M + min(qrow, p.M - 1)) * D + 4 * half_id;
+  floatx4 q[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) q[ks] = *reinterpret_cast<const floatx4*>(qp + 8 * ks);
+
+  floatx16 acc[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) acc[i] = floatx16{};
+  float m_ref = -INFINITY;  // reference max in log2 units
+  float l_run = 0.f;
+  const float c = p.scale_log2;
+
+  for (; t < ntiles; t += NW) {
+    const int k0 = t * BN;
+    // K of this tile has landed; V's DMA is younger
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+    floatx16 part[4] = {};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const floatx4 a = *reinterpret_cast<const floatx4*>(
+          sk + col * ROWB + 16 * ((2 * ks + half_id) ^ (col % CH)));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        part[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], q[ks][j], part[j], 0, 0, 0);
+    }
+    floatx16 s = (part[0] + part[1]) + (part[2] + part[3]);
+    // the stage's reads have completed before the next tile overwrites it
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    dma(kp, t + NW, sk, true);
+
+    if (k0 + BN > min_lim) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (k0 + 8 * (i >> 2) + 4 * half_id + (i & 3) >= lim) s[i] = -INFINITY;
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32)) * c;
+    if (__builtin_amdgcn_ballot_w64(mx > m_ref + kRescaleLog2) != 0) {
+      const float m_new = fmaxf(m_ref, mx);
+      const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int i = 0; i < DB; ++i) acc[i] = acc[i] * alpha;
+      m_ref = m_new;
+    }
+    const float neg_m = m_ref == -INFINITY ? 0.f : -m_ref;
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c, neg_m));
+      sum[i & 3] += s[i];
+    }
+    l_run += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");  // V of this tile
+    floatx16 o[2][DB] = {};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int key = 8 * (i >> 2) + 4 * half_id + (i & 3);
+      const floatv a = *reinterpret_cast<const floatv*>(sv + key * ROWB + 4 * DB * col);
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+        o[i >> 3][d] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d], s[i], o[i >> 3][d], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    dma(vp, t + NW, sv, false);
+#pragma unroll
+    for (int d = 0; d < DB; ++d) acc[d] = (acc[d] + o[0][d]) + o[1][d];
+  }
+
+  // the DMAs past the last tile have an empty range, but they write zeros to
+  // the stage: they land before the epilogue reuses it
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // Each wave leaves its state in its own (drained) stage, rows of D floats
+  // with K's chunk swizzle; then every thread merges 16-byte pieces.
+  const float l_tot = l_run + __shfl_xor(l_run, 32);
+  if (half_id == 0) {
+    s_m[wave][col] = m_ref;
+    s_l[wave][col] = l_tot;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int dim = DB * (8 * (i >> 2) + 4 * half_id + (i & 3));
+    floatv o;
+#pragma unroll
+    for (int d = 0; d < DB; ++d) o[d] = acc[d][i];
+    const int ch = (dim / 4) ^ (col % CH);
+    *reinterpret_cast<floatv*>(sk + col * ROWB + 16 * ch + 4 * (dim & 3)) = o;
+  }
+  __syncthreads();
+  float* op = reinterpret_cast<float*>(p.o) + ((int64_t)b * p.Hq + hq) * p.M * D;
+  for (int e = tid; e < 32 * CH; e += 64 * NW) {
+    const int row = e / CH, ch = e % CH;
+    if (q0 + row >= p.M) break;
+    float m_all = s_m[0][row];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m_all = fmaxf(m_all, s_m[w][row]);
+    float l = 0.f;
+    floatx4 o = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (m_all != -INFINITY) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float a = __builtin_amdgcn_exp2f(s_m[w][row] - m_all);  // a wave without keys: 0
+        l += a * s_l[w][row];
+        o += a * *reinterpret_cast<const floatx4*>(smem + w * 2 * TILE + row * ROWB +
+                                                   16 * (ch ^ (row % CH)));
+      }
+    }
+    // no keys: zeros (flashattention_custom/ops.py:39, 52-59 with slen == 0);
+    // no visible key: 0 * inf = NaN, the fully masked row
+    const float inv = hk < 0 ? __builtin_nanf("") : kv_len == 0 ? 0.f : 1.f / l;
+    *reinterpret_cast<floatx4*>(op + (int64_t)(q0 + row) * D + 4 * ch) = o * inv;
+  }
+}
+
+// The same op for tensors that are not 16-byte aligned (contiguous views at
+// an odd element), in fp32 arithmetic on the vector ALUs.
 // A workgroup takes kF32Rows query rows of one (sequence, q head). Within a
 // wave, the four lanes of a row split the head dimension (lane = 4 * row +
 // part) and sum their partial dot products with two lane exchanges, so all
@@ -1266,6 +1494,25 @@ static PrefillGrid prefill_grid(const AttnParams& p, int D, int ntq, int group, 
 
 hipError_t launch_prefill(const AttnParams& p, int D, int dtype, hipStream_t stream) {
   if (dtype == 1) {
+    // 16-byte loads and LDS DMA need 16-byte aligned rows. B=2, 16 heads,
+    // M = N = 1000, D = 128, causal: 107 us on the matrix cores, 623 us on
+    // the vector ALUs.
+    const bool al16 = (((uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.o) & 15) == 0;
+    if (al16) {
+      F32Grid g;
+      g.ntq = (p.M + 31) / 32;
+      const int units = p.B * p.Hk;
+      g.by_unit = units % 8 == 0 ? 1 : 0;
+      g.units = g.by_unit ? units / 8 : p.B * p.Hq;
+      g.group = g.by_unit ? p.group : 1;
+      const dim3 grid((unsigned)(g.ntq * p.B * p.Hq));
+      const dim3 block(64 * kF32MfmaWaves);
+      if (D == 128)
+        hipLaunchKernelGGL(prefill_f32_mfma_kernel<128>, grid, block, 0, stream, p, g);
+      else
+        hipLaunchKernelGGL(prefill_f32_mfma_kernel<64>, grid, block, 0, stream, p, g);
+      return hipGetLastError();
+    }
     const dim3 grid((unsigned)((p.M + kF32Rows - 1) / kF32Rows), (unsigned)p.Hq, (unsigned)p.B);
     if (D == 128)
       hipLaunchKernelGGL(prefill_f32_kernel<128>, grid, dim3(64 * kF32Waves), 0, stream, p);
