@@ -322,7 +322,7 @@ static int paged_fwd(const void* q, const void* k_pages, const void* v_pages,
     // 367.1 against 368.4 us fused (same-process A/B), the decode kernels
     // rotating q either way.
     if (decode && app->advance && rope_cos == nullptr &&
-        fa::fused_append_ok(B, M, Hq, Hk, heads_per_kv)) {
+        fa::fused_append_ok(B, M, Hq, Hk, heads_per_kv, PS)) {
       // the decode kernels take the new token (fa_decode.hip, APPEND)
       p.app_k = reinterpret_cast<const fa::f16*>(app->k_new);
       p.app_v = reinterpret_cast<const fa::f16*>(app->v_new);
@@ -390,7 +390,7 @@ static int paged_fwd(const void* q, const void* k_pages, const void* v_pages,
       pc.ws_app = pc.ws_units + (Bc + 1);
       // every field decode_variant reads is set before the occupancy query
       pc.dec_rows = cplan.rows;
-      pc.dec_seg_cost = PS % 16 == 0 ? fa::kSegmentCost : 0;
+      pc.dec_seg_cost = PS % 8 == 0 ? fa::kSegmentCost : 0;
       pc.dec_wgs = fa::decode_launch_wgs(cplan, pc, D);
       e = fa::launch_decode(pc, D, (hipStream_t)stream);
     }

@@ -315,8 +315,10 @@ bool use_decode_path(int B, int M, int Hq, int Hk, int heads_per_kv);
 // Whether a paged call with a fused append (one new token per sequence, at
 // position seqlen[b]) runs the append inside the decode kernels: the decode path
 // with at most two 16-row blocks of query rows per KV head (the fused
-// variants keep the new token's fragments in registers beside them).
-bool fused_append_ok(int B, int M, int Hq, int Hk, int heads_per_kv);
+// variants keep the new token's fragments in registers beside them), and the
+// kernel that the call without the append runs, so that the step's result
+// equals the two calls' bit for bit (PS tokens per page).
+bool fused_append_ok(int B, int M, int Hq, int Hk, int heads_per_kv, int PS);
 // seqlen[b] += 1 for b < B (the fused append's advance when the step does
 // not run on the fused decode kernels).
 hipError_t launch_advance_lengths(int32_t* seqlen, int B, hipStream_t stream);

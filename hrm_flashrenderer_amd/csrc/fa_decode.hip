@@ -6,6 +6,11 @@
 // (and k_off + j <= q_off + i when causal), with K/V of head head_map[hq]
 // (flashattention_custom/ops.py:34-60, csrc/flash_attn_sm75.cu:213-425).
 //
+// Two kernels share the split, the partial slots and the combine:
+// decode_kernel (up to 16 query rows per KV head, and pages whose size 8 does
+// not divide) and decode_wide_kernel (more rows, or pages of 8, 24, ...
+// tokens; described at the kernel).
+//
 // Design (HBM-bound; every K/V byte is read once per KV head):
 //  * The work is split evenly: the (sequence, KV head, 16-token group) units
 //    of the whole batch are counted on the device from seqlen, and each of W
@@ -32,6 +37,7 @@
 //    than 2^8. Partial (max, sum, O) of each (segment, workgroup) go to a
 //    workspace; a combine kernel merges the partials of a row in log2 space.
 #include "fa_common.h"
+#include "fa_tile.h"
 
 #include <algorithm>
 #include <atomic>
@@ -82,11 +88,6 @@ struct DecodeRegs {
 // is read exactly once per call, so it should not displace anything in the
 // caches; on MI355X this raises the sustained rate of the page stream by ~10%.
 constexpr int kStreamHint = 2;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);  // raw buffer, dword format (gfx9)
-}
 
 // Per-lane byte offsets of a group's fragments from its first row (loop
 // invariant), with consecutive rows `rowb` bytes apart (2*D inside a page or
@@ -323,6 +324,79 @@ __device__ __forceinline__ SplitRange split_range(const int* units, int B, int H
   return r;
 }
 
+// What every decode workgroup does first: the unit prefix and the head map in
+// LDS, the copies the combine kernel reads (workgroup 0), and the workgroup's
+// range of units, wave-uniform.
+struct DecodeRange {
+  int w;           // piece of the split
+  int u0, u1, b0;  // units [u0, u1), from sequence b0
+};
+
+__device__ __forceinline__ DecodeRange decode_range(const AttnParams& p, int* s_hmap, int* s_units,
+                                                    int* s_part, int* s_keys, int* s_app) {
+  // The piece of the split this workgroup takes. Dispatch places workgroup
+  // blockIdx on XCD blockIdx % 8, so XCD x takes pieces [x * W/8, (x+1) * W/8):
+  // neighbouring pieces (the same KV heads and sequences) share an XCD
+  // (token-major step +1.0 %, cfg4 +0.3 %, cfg3 +-0, same process). The
+  // mapping is a bijection when 8 divides W, else the identity; the combine
+  // kernel needs only the piece index.
+  DecodeRange r;
+  r.w = (gridDim.x & 7) == 0 ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3))
+                             : (int)blockIdx.x;
+  const int W = gridDim.x;
+  const int tid = threadIdx.x;
+
+  // The head map is read once, in the same round trip as the key counts of
+  // the unit prefix (Hq <= kMaxHeads = one head per thread), so a segment's
+  // head scan reads LDS instead of waiting on memory.
+  // (the KV head itself: with kv_pair, a segment's rows are its pair's heads)
+  const int my_hk = tid < p.Hq ? p.kv_head_real(tid) : -1;
+  unit_prefix(p, s_units, s_part, s_keys, s_app);
+  s_hmap[tid] = my_hk;
+  __syncthreads();
+  const int U = s_units[p.B];
+  if (r.w == 0) {
+    for (int b = tid; b <= p.B; b += kDecodeThreads) {
+      p.ws_units[b] = s_units[b];
+      if (s_app != nullptr && b < p.B) p.ws_app[b] = s_app[b];
+      // an advance step whose token the append kernel wrote first: the
+      // combine kernel bumps the lengths from this copy
+      if (s_app == nullptr && p.app_advance && b < p.B) p.ws_app[b] = p.seqlen[b];
+    }
+  }
+  const int P = split_cost_p(p, U, W);
+  const SplitRange range = split_range(s_units, p.B, p.Hk, U, W, P, r.w, p.dec_wdiv);
+  // The range is wave-uniform; the LDS reads it comes from leave it in VGPRs,
+  // and the buffer resources built from it would then be rebuilt per lane
+  // (a readfirstlane loop around every K/V load).
+  r.u0 = __builtin_amdgcn_readfirstlane(range.u0);
+  r.u1 = __builtin_amdgcn_readfirstlane(range.u1);
+  r.b0 = __builtin_amdgcn_readfirstlane(range.b0);
+  return r;
+}
+
+// Query heads that read KV head hk (any head_map, not only h / group), listed
+// in head order by wave 0; ends with a barrier.
+__device__ __forceinline__ void list_heads(const AttnParams& p, int hk, int shift, const int* s_hmap,
+                                           int* s_heads, int* s_count) {
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < 64) {
+    int count = 0;
+    for (int base = 0; base < p.Hq; base += 64) {
+      const int hq = base + lane;
+      const bool match = hq < p.Hq && (s_hmap[hq] >> shift) == hk;
+      const uint64_t mask = __ballot(match);
+      if (match) {
+        const int pos = count + __popcll(mask & ((1ull << lane) - 1ull));
+        if (pos < kMaxHeads) s_heads[pos] = hq;
+      }
+      count += __popcll(mask);
+    }
+    if (lane == 0) *s_count = min(count, kMaxHeads);
+  }
+  __syncthreads();
+}
+
 // Balanced decode. The work is the list of units (sequence b, KV head hk,
 // 16-key group g) in (b, hk, g) order; workgroup w of W takes a contiguous
 // range of it under the cost split above (an equal share of units plus
@@ -342,7 +416,7 @@ __device__ __forceinline__ SplitRange split_range(const int* units, int B, int H
 // a q beyond the fp16 range never becomes inf) and is folded back into the
 // row's score scale.
 //
-// NBLK (1, 2 or 4): column blocks of 16 query rows served by one pass over
+// NBLK: column blocks of 16 query rows served by one pass over
 // the segment's K/V. A KV head with more than 16 * NBLK query rows (heads x
 // positions) is walked once per 16 * NBLK rows.
 //
@@ -374,47 +448,15 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(AttnParams p) {
   __shared__ float s_l[2][kRows];
   __shared__ float s_o[2][kRows][OPAD];
 
-  // The piece of the split this workgroup takes. Dispatch places workgroup
-  // blockIdx on XCD blockIdx % 8, so XCD x takes pieces [x * W/8, (x+1) * W/8):
-  // neighbouring pieces (the same KV heads and sequences) share an XCD
-  // (token-major step +1.0 %, cfg4 +0.3 %, cfg3 +-0, same process). The
-  // mapping is a bijection when 8 divides W, else the identity; the combine
-  // kernel needs only the piece index.
-  const int w = (gridDim.x & 7) == 0
-                    ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3))
-                    : (int)blockIdx.x;
-  const int W = gridDim.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15;       // MFMA column: query row within the block
   const int quarter = lane >> 4; // 0..3
 
-  // The head map is read once, in the same round trip as the key counts of
-  // the unit prefix (Hq <= kMaxHeads = one head per thread), so a segment's
-  // head scan below reads LDS instead of waiting on memory.
-  // (the KV head itself: with kv_pair, a segment's rows are its pair's heads)
-  const int my_hk = tid < p.Hq ? p.kv_head_real(tid) : -1;
-  unit_prefix(p, s_units, s_part, s_keys, APPEND ? s_app : nullptr);
-  s_hmap[tid] = my_hk;
-  __syncthreads();
-  const int U = s_units[p.B];
-  if (w == 0) {
-    for (int b = tid; b <= p.B; b += kDecodeThreads) {
-      p.ws_units[b] = s_units[b];
-      if (APPEND && b < p.B) p.ws_app[b] = s_app[b];
-      // an advance step whose token the append kernel wrote first: the
-      // combine kernel bumps the lengths from this copy
-      if (!APPEND && p.app_advance && b < p.B) p.ws_app[b] = p.seqlen[b];
-    }
-  }
-  const int P = split_cost_p(p, U, W);
-  const SplitRange range = split_range(s_units, p.B, p.Hk, U, W, P, w, p.dec_wdiv);
-  // The range is wave-uniform; the LDS reads it comes from leave it in VGPRs,
-  // and the buffer resources built from it would then be rebuilt per lane
-  // (a readfirstlane loop around every K/V load).
-  const int u0 = __builtin_amdgcn_readfirstlane(range.u0);
-  const int u1 = __builtin_amdgcn_readfirstlane(range.u1);
+  const DecodeRange range =
+      decode_range(p, s_hmap, s_units, s_part, s_keys, APPEND ? s_app : nullptr);
+  const int u0 = range.u0, u1 = range.u1, w = range.w;
   if (u0 >= u1) return;
 
   const f16* qp = reinterpret_cast<const f16*>(p.q);
@@ -484,22 +526,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(AttnParams p) {
     };
     prefetch();
 
-    // Query heads that read KV head hk (any head_map, not only h / group).
-    if (wave == 0) {
-      int count = 0;
-      for (int base = 0; base < p.Hq; base += 64) {
-        const int hq = base + lane;
-        const bool match = hq < p.Hq && (s_hmap[hq] >> (pair ? 1 : 0)) == hk;
-        const uint64_t mask = __ballot(match);
-        if (match) {
-          const int pos = count + __popcll(mask & ((1ull << lane) - 1ull));
-          if (pos < kMaxHeads) s_heads[pos] = hq;
-        }
-        count += __popcll(mask);
-      }
-      if (lane == 0) s_count = min(count, kMaxHeads);
-    }
-    __syncthreads();
+    list_heads(p, hk, pair ? 1 : 0, s_hmap, s_heads, &s_count);
     const int nrows = s_count * p.M;
 
     // NBLK column blocks of 16 query rows share each K/V group load: the K
@@ -785,7 +812,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(AttnParams p) {
   };
 
   // The segments of [u0, u1), from the sequence the split found.
-  int b = __builtin_amdgcn_readfirstlane(range.b0);
+  int b = range.b0;
   for (int u = u0; u < u1;) {
     while (s_units[b + 1] <= u) ++b;
     const int G = fdiv(s_units[b + 1] - s_units[b], p.hk_div);
@@ -798,6 +825,356 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(AttnParams p) {
   }
 }
 
+
+// Decode with 17 and more query rows per KV head, or pages of a multiple of 8
+// tokens that is not one of 16: the same units, split, slots and combine as
+// decode_kernel, on 32-key tiles staged in LDS.
+//
+// The 16x16 tiles of decode_kernel spend a softmax on 4 keys per lane and a
+// half-rate MFMA on PV; with four 16-row blocks (24 sequences of 1024-8192
+// keys, 64/8 heads, M = 5: 390 MB) they took 121 us against 94 here, with two
+// (M = 3) 96 against 91, and M = 8 157 against 113. Pages of 8 tokens had to
+// load row by row (M = 1: 242 us against 88). One 16-row block of whole-group
+// loads stays on decode_kernel (M = 1: 81 us), whose segments start and merge
+// sooner. Here every wave DMAs its own 32-key tiles into
+// two LDS stages of its own (2 x 16 KB at D = 128, no barrier in the loop) and
+// runs the prefill kernel's tile: S^T = K Q^T and O^T = V^T P^T on
+// 32x32x16 MFMAs, the V operand by the transposing LDS read, both operands
+// read once for the NB blocks of 32 rows. K's stage is refilled once QK^T has
+// read it and V's after PV, so 16 to 32 KB per wave are in flight. The tile
+// then costs about a third of the time its bytes take at the streaming rate
+// (NB = 2).
+//  * A tile is two 16-key groups of the wave's range; SL-key slabs (16, or 8
+//    for pages of 8, 24, ...) lie in one page and are one buffer resource each,
+//    whose range ends at the last key, so later rows land as zeros. The page
+//    lookups are scalar loads issued a tile ahead of their use.
+//  * DMAs past the wave's last tile have an empty range. They still write
+//    zeros to their stage, so the segment drains them before it reuses it.
+template <int D, int NB, int SL>
+__global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams p) {
+  using C = DmaCfg<D>;
+  constexpr int BN = 32;
+  constexpr int TILE = BN * C::ROWB;
+  constexpr int KSTEPS = D / 16;
+  constexpr int DBLK = D / 32;
+  constexpr int NSLAB = BN / SL;
+  constexpr int IPS = SL / C::RPI;          // DMA instructions per slab
+  constexpr int NDMA = NSLAB * IPS;         // per tile of K (and of V)
+  constexpr int NM = NB < 2 ? NB : 2;       // blocks merged at a time: they fill the stages
+  constexpr int CF = D / 4;                 // 16-byte chunks of a partial fp32 row
+  static_assert(IPS >= 1, "slab smaller than one wave-wide load");
+  static_assert(NM * 32 * D * 4 <= 4 * TILE, "merge buffer larger than a wave's stages");
+  // a store address the caller's workspace only aligns to 4 bytes
+  typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+
+  __shared__ __attribute__((aligned(1024))) char smem[kDecodeWaves * 4 * TILE];
+  __shared__ int s_hmap[kMaxHeads];
+  __shared__ int s_heads[kMaxHeads];
+  __shared__ int s_count;
+  __shared__ int s_units[kMaxBatch + 1];
+  __shared__ int s_keys[kMaxBatch];
+  __shared__ int s_part[kDecodeWaves];
+  __shared__ float s_m[kDecodeWaves][NB * 32];
+  __shared__ float s_l[kDecodeWaves][NB * 32];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31;       // MFMA column: query row within the block
+  const int half_id = lane >> 5;
+
+  const DecodeRange range = decode_range(p, s_hmap, s_units, s_part, s_keys, nullptr);
+  if (range.u0 >= range.u1) return;
+
+  const f16* qp = reinterpret_cast<const f16*>(p.q);
+  const char* kp = reinterpret_cast<const char*>(p.k);
+  const char* vp = reinterpret_cast<const char*>(p.v);
+  const float c = p.scale_log2;
+  char* stage = smem + wave * 4 * TILE;   // K0 V0 K1 V1
+
+  // byte offsets of this lane's 16 bytes within a slab, per DMA instruction; K's
+  // swizzle also depends on the slab's place in the tile (its parity: CH <= 16)
+  uint32_t vk[2][IPS], vv[IPS];
+#pragma unroll
+  for (int i = 0; i < IPS; ++i) {
+    const int row = C::RPI * i + lane / C::CH, ch = lane % C::CH;
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+      vk[o][i] = (uint32_t)(row * C::ROWB + 16 * (ch ^ C::swz_k(o * SL + row)));
+    vv[i] = (uint32_t)(row * C::ROWB + 16 * (ch ^ C::swz_v(row)));
+  }
+  // operand offsets within a stage, as in the prefill kernel
+  const int gq = lane >> 4, sl = lane & 15;
+  const int vrow = 4 * (gq >> 1) + (sl >> 2);
+  const int kbase = col * C::ROWB + 16 * (half_id ^ C::swz_k(col));
+  const int vd = 16 * (gq & 1) + 4 * (sl & 3);
+  const int vbase = TILE + vrow * C::ROWB + 16 * ((vd >> 3) ^ C::swz_v(vrow)) + 2 * (vd & 7);
+  int kofs[KSTEPS], vofs[DBLK];
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks) kofs[ks] = kbase ^ (32 * ks);
+#pragma unroll
+  for (int i = 0; i < DBLK; ++i) vofs[i] = vbase ^ (64 * i);
+
+  struct TileSrc {
+    int64_t off[NSLAB];
+    uint32_t bytes[NSLAB];
+  };
+
+  // One (b, hk) segment, 16-key groups [g_begin, g_end).
+  auto segment = [&](int b, int hk, int g_begin, int g_end, int slot) {
+    const int qo = p.causal || p.rope_cos != nullptr ? p.q_off(b) : 0;
+    const int ko = p.causal ? p.k_off(b) : 0;
+    const int t_end = __builtin_amdgcn_readfirstlane(min(s_keys[b], g_end << 4));
+    const int ntiles = (g_end - g_begin + 1) >> 1;
+    const int nsteps = ntiles > wave ? (ntiles - wave + kDecodeWaves - 1) / kDecodeWaves : 0;
+    auto tile_key = [&](int k) { return (g_begin << 4) + BN * (wave + kDecodeWaves * k); };
+    auto source = [&](int k) {
+      TileSrc r;
+      const int key = tile_key(k);
+#pragma unroll
+      for (int s = 0; s < NSLAB; ++s) {
+        const int valid = min(SL, t_end - (key + SL * s));
+        const int64_t off = valid > 0 ? p.kv.row_offset(b, hk, key + SL * s) : -1;
+        r.off[s] = off >= 0 ? 2 * off : 0;
+        r.bytes[s] = off >= 0 ? (uint32_t)(valid * C::ROWB) : 0u;
+      }
+      return r;
+    };
+    auto dma_k = [&](const TileSrc& r, int st) {
+#pragma unroll
+      for (int s = 0; s < NSLAB; ++s) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(kp + r.off[s], r.bytes[s]);
+        lds_dma_slab<IPS>(rs, stage + 2 * st * TILE + SL * s * C::ROWB, vk[s & 1]);
+      }
+    };
+    auto dma_v = [&](const TileSrc& r, int st) {
+#pragma unroll
+      for (int s = 0; s < NSLAB; ++s) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(vp + r.off[s], r.bytes[s]);
+        lds_dma_slab<IPS>(rs, stage + (2 * st + 1) * TILE + SL * s * C::ROWB, vv);
+      }
+    };
+
+    // the first tile leaves before the head scan and the Q loads
+    auto dma_tile = [&](int k, int st) {
+      const TileSrc r = source(k);
+      dma_k(r, st);
+      dma_v(r, st);
+    };
+    dma_tile(0, 0);
+    list_heads(p, hk, 0, s_hmap, s_heads, &s_count);
+    const int nrows = s_count * p.M;
+
+    for (int rc0 = 0; rc0 < nrows; rc0 += 32 * NB) {
+      if (rc0 > 0) dma_tile(0, 0);  // a later pass over the same groups
+      bool blk_live[NB];
+      int row_lim[NB];          // keys j < row_lim are visible to this lane's row
+      half8 qreg[NB][KSTEPS];
+      float m_ref[NB], neg_m[NB], thr[NB], l_run[NB];
+      floatx16 acc[NB][DBLK];
+#pragma unroll
+      for (int bk = 0; bk < NB; ++bk) {
+        const int rc = rc0 + 32 * bk;
+        blk_live[bk] = rc < nrows;
+        const bool row_ok = rc + col < nrows;
+        const int ridx = row_ok ? rc + col : 0;
+        const int hi = ridx / p.M;
+        const int qi = ridx - hi * p.M;
+        const int hq = s_heads[hi];
+        const int64_t qoff = (((int64_t)b * p.Hq + hq) * p.M + qi) * D + 8 * half_id;
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          const half8 v = *reinterpret_cast<const half8*>(qp + qoff + 16 * ks);
+          qreg[bk][ks] = row_ok ? v : half8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+        if (p.rope_cos != nullptr && row_ok)
+          rope_fragment<KSTEPS, 16>(qreg[bk], p, qo + qi, 8 * half_id);
+        row_lim[bk] = t_end;
+        if (p.causal) {
+          const int64_t lim = (int64_t)qo + qi - ko + 1;
+          if (lim < t_end) row_lim[bk] = lim < 0 ? 0 : (int)lim;
+        }
+        m_ref[bk] = -INFINITY;
+        neg_m[bk] = 0.f;
+        thr[bk] = -INFINITY;
+        l_run[bk] = 0.f;
+#pragma unroll
+        for (int i = 0; i < DBLK; ++i) acc[bk][i] = floatx16{};
+      }
+      // keys below this are visible to every row
+      int min_lim = t_end;
+      if (p.causal) {
+        const int64_t lim = (int64_t)qo - ko + 1;
+        if (lim < min_lim) min_lim = lim < 0 ? 0 : (int)lim;
+      }
+      const half2v ones = half2v{(f16)1.f, (f16)1.f};
+      // Q has arrived, as the compiler sees too: its waits for Q then come
+      // before the second tile's DMAs and not after them
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+      dma_tile(1, 1);
+
+      auto step = [&](auto par, int k) {
+        constexpr int ST = decltype(par)::value;
+        const char* buf = stage + 2 * ST * TILE;
+        const int k0 = tile_key(k);
+        const TileSrc next = source(k + 2);
+        // in flight, oldest first: K and V of tile k, then of tile k + 1
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NDMA) : "memory");
+        floatx16 s[NB];
+#pragma unroll
+        for (int bk = 0; bk < NB; ++bk) s[bk] = floatx16{};
+        constexpr int KA = 2;  // operands read ahead
+        half8 ka[KA];
+#pragma unroll
+        for (int i = 0; i < KA; ++i) ka[i] = *reinterpret_cast<const half8*>(buf + kofs[i]);
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+#pragma unroll
+          for (int bk = 0; bk < NB; ++bk)
+            s[bk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks % KA], qreg[bk][ks], s[bk], 0, 0, 0);
+          if (ks + KA < KSTEPS) ka[ks % KA] = *reinterpret_cast<const half8*>(buf + kofs[ks + KA]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // K's reads have completed before its stage is overwritten
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        dma_k(next, ST);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NDMA) : "memory");  // V of tile k
+        constexpr int NMF = 2 * DBLK;
+        constexpr int VA = 4;
+        half8 va[VA];
+#pragma unroll
+        for (int m = 0; m < VA; ++m) va[m] = ld_vt<D>(buf, vofs, m / DBLK, m % DBLK);
+        half8 pb[NB][2];
+#pragma unroll
+        for (int bk = 0; bk < NB; ++bk) {
+          if (NB > 2 && !blk_live[bk]) continue;
+          if (k0 + BN > min_lim) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              if (k0 + 8 * (r >> 2) + 4 * half_id + (r & 3) >= row_lim[bk]) s[bk][r] = -INFINITY;
+          }
+          float mx = max16(s[bk]);
+          if (__builtin_amdgcn_ballot_w64(mx > thr[bk]) != 0) {
+            mx = fmaxf(mx, __shfl_xor(mx, 32)) * c;
+            const float m_new = fmaxf(m_ref[bk], mx);
+            const float alpha =
+                m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_ref[bk] - m_new);
+            l_run[bk] *= alpha;
+#pragma unroll
+            for (int i = 0; i < DBLK; ++i) acc[bk][i] = acc[bk][i] * alpha;
+            m_ref[bk] = m_new;
+            neg_m[bk] = m_new == -INFINITY ? 0.f : -m_new;
+            thr[bk] = (m_new + kRescaleLog2) / c;
+          }
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            pb[bk][0][j] = (f16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[bk][j], c, neg_m[bk]));
+            pb[bk][1][j] = (f16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[bk][8 + j], c, neg_m[bk]));
+          }
+#pragma unroll
+          for (int st = 0; st < 2; ++st) {
+#pragma unroll
+            for (int j = 0; j < 8; j += 2)
+              l_run[bk] = __builtin_amdgcn_fdot2(half2v{pb[bk][st][j], pb[bk][st][j + 1]}, ones,
+                                                 l_run[bk], false);
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < NMF; ++m) {
+          const int st = m / DBLK, i = m % DBLK;
+#pragma unroll
+          for (int bk = 0; bk < NB; ++bk) {
+            if (NB <= 2 || blk_live[bk])
+              acc[bk][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[m % VA], pb[bk][st], acc[bk][i], 0, 0, 0);
+          }
+          if (m + VA < NMF) va[m % VA] = ld_vt<D>(buf, vofs, (m + VA) / DBLK, (m + VA) % DBLK);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        dma_v(next, ST);
+      };
+      for (int k = 0; k < nsteps; k += 2) {
+        step(std::integral_constant<int, 0>{}, k);
+        if (k + 1 < nsteps) step(std::integral_constant<int, 1>{}, k + 1);
+      }
+      // the DMAs past the last tile write zeros to the stages reused below
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+      // Merge of the four waves' states, NM blocks at a time: each wave
+      // leaves rows of D floats (16-byte chunks swizzled by the row) in its
+      // own stages, then every thread sums 16-byte pieces over the waves.
+#pragma unroll
+      for (int bk = 0; bk < NB; ++bk) {
+        const float l_tot = l_run[bk] + __shfl_xor(l_run[bk], 32);
+        if (half_id == 0) {
+          s_m[wave][32 * bk + col] = m_ref[bk];
+          s_l[wave][32 * bk + col] = l_tot;
+        }
+      }
+#pragma unroll
+      for (int b0 = 0; b0 < NB; b0 += NM) {
+        if (rc0 + 32 * b0 >= nrows) break;
+        if (b0 > 0) __syncthreads();  // the previous blocks have been read
+#pragma unroll
+        for (int j = 0; j < NM; ++j) {
+#pragma unroll
+          for (int i = 0; i < DBLK; ++i) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              const floatx16& a = acc[b0 + j][i];
+              *reinterpret_cast<floatx4*>(stage + (32 * j + col) * 4 * D +
+                                          16 * ((8 * i + 2 * g + half_id) ^ (col % CF))) =
+                  floatx4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+            }
+          }
+        }
+        __syncthreads();
+        for (int e = tid; e < NM * 32 * CF; e += kDecodeThreads) {
+          const int row = e / CF, ch = e % CF;
+          const int lr = 32 * b0 + row;      // row of the pass
+          const int ri = rc0 + lr;           // row of the slot
+          if (ri >= nrows || ri >= p.dec_rows) continue;  // rows past the slot: NaN in the combine
+          float mx = s_m[0][lr];
+#pragma unroll
+          for (int w = 1; w < kDecodeWaves; ++w) mx = fmaxf(mx, s_m[w][lr]);
+          float lsum = 0.f;
+          floatx4 osum = floatx4{0.f, 0.f, 0.f, 0.f};
+          if (mx != -INFINITY) {
+#pragma unroll
+            for (int w = 0; w < kDecodeWaves; ++w) {
+              const float a = __builtin_amdgcn_exp2f(s_m[w][lr] - mx);
+              lsum += a * s_l[w][lr];
+              osum += a * *reinterpret_cast<const floatx4*>(smem + w * 4 * TILE + row * 4 * D +
+                                                            16 * (ch ^ (row % CF)));
+            }
+          }
+          const int64_t srow = (int64_t)slot * p.dec_rows + ri;
+          *reinterpret_cast<floatx4u*>(p.ws_o + srow * D + 4 * ch) = osum;
+          if (ch == 0) {
+            p.ws_ml[srow * 2 + 0] = mx;
+            p.ws_ml[srow * 2 + 1] = lsum;
+          }
+        }
+      }
+      __syncthreads();  // the stages, s_m and s_l are free again
+    }
+    if (nrows == 0) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+  };
+
+  int b = range.b0;
+  for (int u = range.u0; u < range.u1;) {
+    while (s_units[b + 1] <= u) ++b;
+    const int G = fdiv(s_units[b + 1] - s_units[b], p.hk_div);
+    const int rel = u - s_units[b];
+    const int hk = rel / G;
+    const int g_lo = rel - hk * G;
+    const int uend = min(range.u1, s_units[b] + (hk + 1) * G);
+    segment(b, hk, g_lo, g_lo + (uend - u), b * p.Hk + hk + range.w);
+    u = uend;
+  }
+}
 
 // The fused append's page writes, done by workgroups of the combine grid of
 // their own (after the merge workgroups), so that their load -> page lookup
@@ -996,28 +1373,47 @@ __global__ __launch_bounds__(WIDE ? 64 * kWideWaves : 256) void decode_combine_k
   }
 }
 
-// The decode kernel variant a call runs: row loads from whole 16-token
-// groups (ALIGNED: pages of a multiple of 16 tokens, or unpaged rows at a
-// fixed stride whose 16-row span fits a buffer range), the fp32-query split
-// (the token-major entry, one row block per pass), and the row blocks served
-// per K/V pass: enough 16-row blocks for a KV head's query rows
-// (heads_per_kv * M = dec_rows), up to 4.
+// The decode kernel variant a call runs.
+//  * wide_nb > 0: decode_wide_kernel with that many 32-row blocks per pass and
+//    slabs of wide_sl keys (decode_is_wide).
+//  * else decode_kernel: row loads from whole 16-token groups (aligned: pages
+//    of a multiple of 16 tokens, or unpaged rows at a fixed stride whose
+//    16-row span fits a buffer range) or one by one, the fp32-query split
+//    (the token-major entry), the fused append, and the 16-row blocks served
+//    per K/V pass: one, or for rows loaded one by one enough for the KV head's
+//    query rows (heads_per_kv * M = dec_rows), up to 4 (2 at D = 128, whose
+//    four blocks spill).
 struct DecodeVariant {
+  int wide_nb;
+  int wide_sl;
   bool aligned;
   bool qsplit;
   int nblk;
-  bool append;  // fused append (at most two row blocks: fused_append_ok)
+  bool append;
 };
 
-// Row blocks per pass: four (64 rows), except the per-row load variant at
-// D = 128, whose four blocks spill; it walks larger groups in passes of 32
-// rows. At D = 128 the four-block variant keeps one 16-key group in flight
-// per wave (their O accumulators alone take 128 registers).
-constexpr int max_row_blocks(int D, bool aligned) { return D == 128 && !aligned ? 2 : 4; }
+constexpr int max_row_blocks(int D) { return D == 128 ? 2 : 4; }
+// four 32-row blocks spill at D = 128
+constexpr int max_wide_blocks(int D) { return D == 128 ? 2 : 4; }
+
+// Whether the 32-key LDS tiles serve a call with `rows` query rows per KV head:
+// contiguous K/V or pages of whole 8-key slabs, and either more rows than one
+// 16-row block or pages that the whole-group loads of decode_kernel cannot take.
+bool decode_is_wide(bool paged, int PS, int rows) {
+  if (paged && PS % 8 != 0) return false;
+  return rows > kRows || (paged && PS % 16 != 0);
+}
 
 DecodeVariant decode_variant(const AttnParams& p) {
-  DecodeVariant v;
+  DecodeVariant v = {};
   v.qsplit = p.q_f32 != 0;
+  v.append = p.app_k != nullptr;
+  if (!v.qsplit && !v.append && (p.kv.paged || p.kv.stride_tok == p.kv.D) &&
+      decode_is_wide(p.kv.paged, p.kv.PS, p.dec_rows)) {
+    v.wide_nb = p.dec_rows <= 32 ? 1 : p.dec_rows <= 64 ? 2 : max_wide_blocks(p.kv.D);
+    v.wide_sl = p.kv.paged && p.kv.PS % 16 != 0 ? 8 : 16;
+    return v;
+  }
   // Unpaged rows D apart (contiguous K/V), or, with the fp32 query split
   // (whose variant takes the row stride at run time), any stride whose 16-row
   // span fits a 32-bit buffer range.
@@ -1025,29 +1421,34 @@ DecodeVariant decode_variant(const AttnParams& p) {
             : v.qsplit   ? p.kv.stride_tok >= p.kv.D && p.kv.stride_tok <= ((int64_t)1 << 24)
                          : p.kv.stride_tok == p.kv.D;
   const int want = p.dec_rows <= kRows ? 1 : p.dec_rows <= 2 * kRows ? 2 : 4;
-  v.nblk = v.qsplit ? 1 : std::min(want, max_row_blocks(p.kv.D, v.aligned));
-  v.append = p.app_k != nullptr;
+  v.nblk = v.qsplit || v.aligned ? 1 : std::min(want, max_row_blocks(p.kv.D));
   return v;
 }
 
-template <int D, bool ALIGNED>
-const void* decode_fn_rows(int nblk, bool append) {
-  constexpr int NB4 = max_row_blocks(D, ALIGNED) >= 4 ? 4 : 2;
-  if (append)
-    return nblk == 1 ? reinterpret_cast<const void*>(&decode_kernel<D, ALIGNED, false, 1, true>)
-                     : reinterpret_cast<const void*>(&decode_kernel<D, ALIGNED, false, 2, true>);
-  return nblk == 1 ? reinterpret_cast<const void*>(&decode_kernel<D, ALIGNED, false, 1, false>)
-       : nblk == 2 ? reinterpret_cast<const void*>(&decode_kernel<D, ALIGNED, false, 2, false>)
-                   : reinterpret_cast<const void*>(&decode_kernel<D, ALIGNED, false, NB4, false>);
+template <int D, int SL>
+const void* decode_wide_fn(int nb) {
+  return nb == 1 ? reinterpret_cast<const void*>(&decode_wide_kernel<D, 1, SL>)
+       : nb == 2 ? reinterpret_cast<const void*>(&decode_wide_kernel<D, 2, SL>)
+                 : reinterpret_cast<const void*>(&decode_wide_kernel<D, max_wide_blocks(D), SL>);
 }
 
 template <int D>
 const void* decode_fn(DecodeVariant v) {
+  if (v.wide_nb > 0)
+    return v.wide_sl == 16 ? decode_wide_fn<D, 16>(v.wide_nb) : decode_wide_fn<D, 8>(v.wide_nb);
   if (v.qsplit)
     return v.aligned ? reinterpret_cast<const void*>(&decode_kernel<D, true, true, 1, false>)
                      : reinterpret_cast<const void*>(&decode_kernel<D, false, true, 1, false>);
-  return v.aligned ? decode_fn_rows<D, true>(v.nblk, v.append)
-                   : decode_fn_rows<D, false>(v.nblk, v.append);
+  if (v.aligned)
+    return v.append ? reinterpret_cast<const void*>(&decode_kernel<D, true, false, 1, true>)
+                    : reinterpret_cast<const void*>(&decode_kernel<D, true, false, 1, false>);
+  constexpr int NBMAX = max_row_blocks(D);
+  if (v.append)
+    return v.nblk == 1 ? reinterpret_cast<const void*>(&decode_kernel<D, false, false, 1, true>)
+                       : reinterpret_cast<const void*>(&decode_kernel<D, false, false, 2, true>);
+  return v.nblk == 1 ? reinterpret_cast<const void*>(&decode_kernel<D, false, false, 1, false>)
+       : v.nblk == 2 ? reinterpret_cast<const void*>(&decode_kernel<D, false, false, 2, false>)
+                     : reinterpret_cast<const void*>(&decode_kernel<D, false, false, NBMAX, false>);
 }
 
 int decode_grid_wgs(int D, DecodeVariant var) {
@@ -1062,9 +1463,12 @@ int decode_grid_wgs(int D, DecodeVariant var) {
   static std::atomic<int> cache[64][64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  const int blk = var.nblk == 1 ? 0 : var.nblk == 2 ? 1 : 2;
-  const int idx = (var.append ? 32 : 0) + (D == 128 ? 16 : 0) + blk * 4 + (var.qsplit ? 2 : 0) +
-                  (var.aligned ? 1 : 0);
+  // 0..47: decode_kernel, 24 per head dim; 48..63: decode_wide_kernel, 8 per head dim
+  const int blk = var.nblk <= 1 ? 0 : var.nblk == 2 ? 1 : 2;
+  const int idx = var.wide_nb > 0
+                      ? 48 + (D == 128 ? 8 : 0) + (var.wide_sl == 8 ? 4 : 0) + var.wide_nb / 2
+                      : (D == 128 ? 24 : 0) + (var.append ? 12 : 0) + blk * 4 +
+                            (var.qsplit ? 2 : 0) + (var.aligned ? 1 : 0);
   int v = cache[dev][idx].load(std::memory_order_relaxed);
   if (v > 0) return v;
   int cus = 0, per_cu = 0;
@@ -1105,10 +1509,10 @@ bool use_decode_path(int B, int M, int Hq, int Hk, int heads_per_kv) {
   return rows <= 4 * kRows || (packable && rows <= 16 * kRows);
 }
 
-bool fused_append_ok(int B, int M, int Hq, int Hk, int heads_per_kv) {
+bool fused_append_ok(int B, int M, int Hq, int Hk, int heads_per_kv, int PS) {
   if (!use_decode_path(B, M, Hq, Hk, heads_per_kv)) return false;
   const int64_t hpk = heads_per_kv <= 0 || heads_per_kv > Hq ? Hq : heads_per_kv;
-  return hpk * M <= 2 * kRows;
+  return hpk * M <= 2 * kRows && !decode_is_wide(true, PS, (int)(hpk * M));
 }
 
 int decode_launch_wgs(const DecodePlan& plan, const AttnParams& p, int D) {

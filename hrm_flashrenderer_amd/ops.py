@@ -504,7 +504,7 @@ def flash_attn_paged_append(q, k_pages, v_pages, k_new, v_new, seqlen, page_size
     The reference's decode step makes these two calls (cache.append,
     engine/llama_tp.py:65-78, then flash_attn_paged, :186-200). Here, with
     start_pos=None and no rope, when the attention runs on the decode kernels
-    with at most 32 query rows per KV head (single-token decode at the
+    with at most 16 query rows per KV head (single-token decode at the
     benchmark shapes), the append has no launch of its own. The new token is
     every sequence's last key: the decode kernel reads it from k_new / v_new,
     and its merge kernel writes it into the pages. Other calls (rope steps

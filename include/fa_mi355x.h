@@ -278,8 +278,10 @@ int fa_paged_kv_scatter(void* k_pages, void* v_pages, const void* k_new, const v
  *                 as fa_paged_kv_append_rope does, Q at q_off(b) + i.
  *   workspace : as for fa_flash_attn_paged_fwd (fa_paged_workspace_bytes).
  * With advance = 1, when the attention runs on the decode kernels with at
- * most 32 query rows per KV head (heads_per_kv * M <= 32: single-token
- * decode at the benchmark shapes), the append costs no launch of its own:
+ * most 16 query rows per KV head (heads_per_kv * M <= 16: single-token
+ * decode at the benchmark shapes; 32 when 8 does not divide the page size) and
+ * pages that are not of 8, 24, 40, ... tokens, the append costs no launch of
+ * its own:
  * the new token is every sequence's last key, and the decode kernel takes
  * its row from k_new / v_new (rotated there with rotary tables). The merge
  * kernel, which runs after every page read, writes the row into the pages
