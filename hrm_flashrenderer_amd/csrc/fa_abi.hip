@@ -241,6 +241,10 @@ static int contig_fwd(const void* q, const void* k, const void* v, void* o, int 
     }
     return launch_status(e);
   }
+  if (decode_ok) {
+    p.ws = workspace;
+    p.ws_bytes = workspace_bytes;
+  }
   return launch_status(fa::launch_prefill(p, D, dtype, (hipStream_t)stream));
 }
 
@@ -399,6 +403,8 @@ static int paged_fwd(const void* q, const void* k_pages, const void* v_pages,
     // the prefill kernel packs the rows of a KV head's q heads (at most
     // heads_per_kv of them) into shared 128-row tiles when M < 128
     p.pack_heads = heads_per_kv > 0 ? std::min(heads_per_kv, Hq) : 0;
+    p.ws = workspace;
+    p.ws_bytes = workspace_bytes;
     e = fa::launch_prefill(p, D, FA_DTYPE_F16, (hipStream_t)stream);
   }
   // the decode path's combine kernel advances the lengths itself (from the

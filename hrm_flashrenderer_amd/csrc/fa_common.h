@@ -170,6 +170,9 @@ struct AttnParams {
   const f16* app_v;
   int app_advance;               // 0 or 1
   int* ws_app;                   // [B] positions the decode kernel publishes to the combine kernel
+  // prefill: the caller's workspace (nullable), for a split of the keys
+  void* ws;
+  size_t ws_bytes;
 
   __device__ __forceinline__ int q_off(int b) const { return q_offsets ? q_offsets[b] : q_offset; }
   __device__ __forceinline__ int k_off(int b) const { return k_offsets ? k_offsets[b] : k_offset; }

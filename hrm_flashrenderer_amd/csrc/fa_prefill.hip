@@ -33,6 +33,7 @@
 #include "fa_tile.h"
 
 
+#include <algorithm>
 #include <type_traits>
 
 namespace fa {
@@ -43,6 +44,9 @@ constexpr int kBM = 128;     // query rows per workgroup
 constexpr int kMaxPackHeads = 256;  // q heads listed per KV head in the packed layout
 constexpr int kBN = 64;      // keys per tile
 constexpr int kThreads = 256;
+constexpr int kSlots = 768;         // resident workgroups of prefill_b32_kernel: 3 per CU, 256 CUs
+constexpr int kSplitMinTiles = 16;  // 32-key tiles of a piece at least
+constexpr int kSplitFrom = 48;      // tiles of an item from which its keys are split
 
 __device__ __forceinline__ uint32_t pack_lo(uint32_t x, uint32_t y) {
   return __builtin_amdgcn_perm(y, x, 0x05040100u);
@@ -347,6 +351,8 @@ struct PrefillGrid {
   int order, kp, tp, head_items, rank;
   int per_pair, ngroups, band, gsz;
   FastDiv d_pair, d_group, d_ngroups, d_band, d_gsz;
+  int slots, pieces;  // workgroups without a split; pieces per item with one
+  FastDiv d_slots;
 };
 
 struct SeqData {
@@ -550,7 +556,23 @@ __device__ __forceinline__ void dma_slab(const QuarterSrc& q, const uint32_t* vo
 // the per-head layout would fill 16 of 128 rows and stream the K/V once per
 // q head). `ntq` is then the number of 128-row tiles per pair, `group` 1,
 // and slot L runs pair L / ntq (consecutive pairs go to different XCDs).
-template <int D, bool PACKED>
+//
+// Split keys. A grid of fewer items than the device's 768 workgroup slots (one
+// sequence's chunk: 256 items at 64 heads x 512 rows) leaves CUs with one
+// workgroup or none. kSplit runs `pieces` workgroups per item, each over an
+// equal share of the item's key tiles (kSplitMinTiles or more; an item of fewer
+// than kSplitFrom tiles is one piece, which finishes it); a piece leaves its unscaled O (fp32),
+// reference max and row sum in the workspace, in the order its lanes hold
+// them (1 KB per store). kMerge is the same item decode on one workgroup per
+// item: it loads the pieces' states, merges them in log2 space and runs the
+// common epilogue.
+// One sequence, 64/8 heads, D = 128, 16-token pages, unsplit -> split: 512 rows
+// over 16000 cached keys 329 -> 272 us (1000 TFLOP/s; a grid that fills the
+// slots by itself runs at 1130), 128 rows 304 -> 105 us, 64 rows (packed) 311
+// -> 90 us; 32/8 heads, D = 64, 512 rows over 8000 keys 127 -> 63 us.
+enum PrefillMode { kWhole, kSplit, kMerge };
+
+template <int D, bool PACKED, int MODE>
 __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, PrefillGrid g) {
   using C = DmaCfg<D>;
   constexpr int BN = 32;
@@ -576,7 +598,8 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
   __shared__ int s_bad[kPackList];
   __shared__ int s_pk_n[2];
 
-  const int slot = blockIdx.x;
+  const int piece = MODE == kSplit ? fdiv((int)blockIdx.x, g.d_slots) : 0;
+  const int slot = (int)blockIdx.x - piece * g.slots;
   const int item = PACKED ? slot : (slot & 7) * g.per_xcd + (slot >> 3);
   if (item >= g.total) return;
   const int group = g.group;
@@ -717,13 +740,16 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
   const int64_t qoff = (int64_t)min(qrow, p.M - 1) * D + 8 * half_id;
   const bool q_ok = qrow < p.M && row_exists;
   half8 qreg[KSTEPS];
+  if constexpr (MODE != kMerge) {
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) {
-    const half8 v = *reinterpret_cast<const half8*>(qp + qoff + 16 * ks);
-    qreg[ks] = q_ok ? v : half8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const half8 v = *reinterpret_cast<const half8*>(qp + qoff + 16 * ks);
+      qreg[ks] = q_ok ? v : half8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
   }
   using Table = SlabTable<D, NW, BN>;
-  const typename Table::RowReq req0 = Table::row_load(p, b, lane, wave);
+  typename Table::RowReq req0;
+  if constexpr (MODE == kWhole) req0 = Table::row_load(p, b, lane, wave);
   const SeqData sd = seq_data(p, b, hq, hk_pair);
   const int hk = PACKED ? hk_pair : pre ? hk_pre : sd.hk;
   const int kv_len = pre ? kv_len_pre : sd.kv_len;
@@ -733,7 +759,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
   const bool head_ok = hk >= 0;
   Table pages;
   pages.base = 0;
-  pages.rows = Table::row_finish(p, b, req0);
+  if constexpr (MODE == kWhole) pages.rows = Table::row_finish(p, b, req0);
   pages.hk_rows = head_ok ? (uint32_t)((int64_t)hk * (p.kv.stride_hk / D)) : 0u;
 
   int wg_lim, wave_lim_max, wave_lim_min;
@@ -769,27 +795,41 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
     wave_lim_max = wave_rows ? row_key_limit(kv_len, p.causal, qo, ko, wrow1) : 0;
     wave_lim_min = wave_rows ? row_key_limit(kv_len, p.causal, qo, ko, wrow0) : 0;
   }
-  const int ntiles = (wg_lim + BN - 1) / BN;
+  // This workgroup's key tiles [t0, ntiles).
+  int ntiles = (wg_lim + BN - 1) / BN;
   const int lim = row_key_limit(kv_len, p.causal, qo, ko, qrow);
+  int t0 = 0, parts = 1;
+  if constexpr (MODE != kWhole) {
+    parts = ntiles < kSplitFrom ? 1 : min(g.pieces, ntiles / kSplitMinTiles);
+    if (MODE == kMerge ? parts == 1 : piece >= parts) return;
+    if constexpr (MODE == kSplit) {
+      t0 = piece * ntiles / parts;
+      ntiles = (piece + 1) * ntiles / parts;
+      pages.fill(p, b, wave, lane, t0);
+    }
+  }
 
   const char* kp = reinterpret_cast<const char*>(p.k);
   const char* vp = reinterpret_cast<const char*>(p.v);
   const SlabLane<D, NW, BN> dl = slab_lane<D, NW, BN>(wave, lane);
-  if (ntiles > 0) {
-    const QuarterSrc s0 = pages.get(p, b, 0, kv_len, wave, lane);
-    dma_slab<D, NW, BN, PACKED>(s0, dl.vk, kp, wave, smem);
-    dma_slab<D, NW, BN, PACKED>(s0, dl.vv, vp, wave, smem + TILE);
-  }
-  if constexpr (NST == 3) {
-    if (ntiles > 1) {
-      const QuarterSrc s1 = pages.get(p, b, 1, kv_len, wave, lane);
-      dma_slab<D, NW, BN, PACKED>(s1, dl.vk, kp, wave, smem + 2 * TILE);
-      dma_slab<D, NW, BN, PACKED>(s1, dl.vv, vp, wave, smem + 3 * TILE);
+  QuarterSrc next_src = QuarterSrc{0, 0u};
+  if constexpr (MODE != kMerge) {
+    if (t0 < ntiles) {
+      const QuarterSrc s0 = pages.get(p, b, t0, kv_len, wave, lane);
+      dma_slab<D, NW, BN, PACKED>(s0, dl.vk, kp, wave, smem);
+      dma_slab<D, NW, BN, PACKED>(s0, dl.vv, vp, wave, smem + TILE);
     }
-  }
-  QuarterSrc next_src = pages.get(p, b, NST - 1, kv_len, wave, lane);
+    if constexpr (NST == 3) {
+      if (t0 + 1 < ntiles) {
+        const QuarterSrc s1 = pages.get(p, b, t0 + 1, kv_len, wave, lane);
+        dma_slab<D, NW, BN, PACKED>(s1, dl.vk, kp, wave, smem + 2 * TILE);
+        dma_slab<D, NW, BN, PACKED>(s1, dl.vv, vp, wave, smem + 3 * TILE);
+      }
+    }
+    next_src = pages.get(p, b, t0 + NST - 1, kv_len, wave, lane);
 
-  if (p.rope_cos != nullptr && q_ok) rope_fragment<KSTEPS, 16>(qreg, p, qo + qrow, 8 * half_id);
+    if (p.rope_cos != nullptr && q_ok) rope_fragment<KSTEPS, 16>(qreg, p, qo + qrow, 8 * half_id);
+  }
 
   // LDS byte offsets of the lane's operands. K: row col, logical chunk
   // 2*ks + half_id at chunk ^ swz_k(col); the chunk bits of 2*ks and half_id
@@ -923,7 +963,8 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
     }
     __builtin_amdgcn_s_setprio(0);
   };
-  for (int t = 0; t < ntiles; t += NST) {
+  // (kMerge: t0 = 0 and ntiles are the whole item's; its pieces ran them)
+  for (int t = MODE == kMerge ? ntiles : t0; t < ntiles; t += NST) {
     step(std::integral_constant<int, 0>{}, t);
     if (t + 1 < ntiles) step(std::integral_constant<int, 1>{}, t + 1);
     if constexpr (NST == 3) {
@@ -938,45 +979,92 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
   // each of 32 rows (with the non-temporal store below: +4.5 % on cfg2).
   // Lane (col, half) holds d = 32i + 8g + 4*half + 0..3 of its row, i.e.
   // half of 16-byte chunk 4i + g.
-  const float l_tot = l_run + __shfl_xor(l_run, 32);
+  float l_tot = l_run + __shfl_xor(l_run, 32);
+  if constexpr (MODE != kWhole) {
+    // the states of an item's pieces, in the lanes' order; the caller's
+    // workspace is only aligned to 4 bytes
+    typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int kStateO = kThreads * 16 * DBLK;  // floats of O per piece
+    const int64_t first = (int64_t)slot * g.pieces;
+    auto o_at = [&](int j) { return p.ws_o + (first + j) * kStateO + (wave * 4 * DBLK * 64 + lane) * 4; };
+    auto ml_at = [&](int j) { return p.ws_ml + ((first + j) * kThreads + tid) * 2; };
+    if constexpr (MODE == kSplit) {
+      if (parts > 1) {
+        float* o = o_at(piece);
+#pragma unroll
+        for (int i = 0; i < DBLK; ++i) {
+#pragma unroll
+          for (int gr = 0; gr < 4; ++gr)
+            *reinterpret_cast<floatx4u*>(o + (4 * i + gr) * 256) =
+                floatx4u{acc_o[i][4 * gr], acc_o[i][4 * gr + 1], acc_o[i][4 * gr + 2],
+                         acc_o[i][4 * gr + 3]};
+        }
+        ml_at(piece)[0] = m_ref;
+        ml_at(piece)[1] = l_tot;
+      }
+    } else {
+      float m_all = -INFINITY;
+      for (int j = 0; j < parts; ++j) m_all = fmaxf(m_all, ml_at(j)[0]);
+      l_tot = 0.f;
+      for (int j = 0; j < parts; ++j) {
+        // a piece whose keys the row does not see has the max -inf: weight 0
+        const float m = ml_at(j)[0];
+        const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_all);
+        l_tot += w * ml_at(j)[1];
+        const float* o = o_at(j);
+#pragma unroll
+        for (int i = 0; i < DBLK; ++i) {
+#pragma unroll
+          for (int gr = 0; gr < 4; ++gr) {
+            const floatx4u x = *reinterpret_cast<const floatx4u*>(o + (4 * i + gr) * 256);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc_o[i][4 * gr + r] += w * x[r];
+          }
+        }
+      }
+    }
+  }
+  const bool finish = MODE != kSplit || parts == 1;
   const float inv = !head_ok ? __builtin_nanf("") : kv_len == 0 ? 0.f : 1.f / l_tot;
   const bool live = qrow < qlen && row_exists;  // padding rows are zeros whatever their Q held
   __syncthreads();  // every wave has finished reading the last K/V stage
-  const int lrow = rblk * 32 + col;
+  if (finish) {
+    const int lrow = rblk * 32 + col;
 #pragma unroll
-  for (int i = 0; i < DBLK; ++i) {
+    for (int i = 0; i < DBLK; ++i) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      half4 h = half4{(f16)(acc_o[i][4 * g + 0] * inv), (f16)(acc_o[i][4 * g + 1] * inv),
-                      (f16)(acc_o[i][4 * g + 2] * inv), (f16)(acc_o[i][4 * g + 3] * inv)};
-      if (!live) h = half4{0, 0, 0, 0};
-      const int chunk = (4 * i + g) ^ C::swz_k(lrow);
-      *reinterpret_cast<half4*>(smem + lrow * C::ROWB + 16 * chunk + 8 * half_id) = h;
+      for (int g = 0; g < 4; ++g) {
+        half4 h = half4{(f16)(acc_o[i][4 * g + 0] * inv), (f16)(acc_o[i][4 * g + 1] * inv),
+                        (f16)(acc_o[i][4 * g + 2] * inv), (f16)(acc_o[i][4 * g + 3] * inv)};
+        if (!live) h = half4{0, 0, 0, 0};
+        const int chunk = (4 * i + g) ^ C::swz_k(lrow);
+        *reinterpret_cast<half4*>(smem + lrow * C::ROWB + 16 * chunk + 8 * half_id) = h;
+      }
+    }
+    __syncthreads();
+    const int rows = min(kBM, (PACKED ? pk_rows : p.M) - q0);
+    f16* ob = op + (int64_t)q0 * D;
+    for (int e = tid; e < rows * C::CH; e += kThreads) {
+      const int r = e / C::CH, ch = e % C::CH;
+      const half8 v = *reinterpret_cast<const half8*>(smem + r * C::ROWB + 16 * (ch ^ C::swz_k(r)));
+      f16* dst;
+      if constexpr (PACKED) {
+        const int pr = q0 + r, j = pr / p.M;
+        dst = reinterpret_cast<f16*>(p.o) + (((int64_t)b * p.Hq + s_pk[j]) * p.M + (pr - j * p.M)) * D;
+      } else {
+        dst = ob + (int64_t)r * D;
+      }
+      // O is not read again by this kernel: a non-temporal store keeps the
+      // K/V lines that other workgroups still read in L2.
+      __builtin_nontemporal_store(v, reinterpret_cast<half8*>(dst + 8 * ch));
     }
   }
-  __syncthreads();
-  const int rows = min(kBM, (PACKED ? pk_rows : p.M) - q0);
-  f16* ob = op + (int64_t)q0 * D;
-  for (int e = tid; e < rows * C::CH; e += kThreads) {
-    const int r = e / C::CH, ch = e % C::CH;
-    const half8 v = *reinterpret_cast<const half8*>(smem + r * C::ROWB + 16 * (ch ^ C::swz_k(r)));
-    f16* dst;
-    if constexpr (PACKED) {
-      const int pr = q0 + r, j = pr / p.M;
-      dst = reinterpret_cast<f16*>(p.o) + (((int64_t)b * p.Hq + s_pk[j]) * p.M + (pr - j * p.M)) * D;
-    } else {
-      dst = ob + (int64_t)r * D;
-    }
-    // O is not read again by this kernel: a non-temporal store keeps the
-    // K/V lines that other workgroups still read in L2.
-    __builtin_nontemporal_store(v, reinterpret_cast<half8*>(dst + 8 * ch));
-  }
-  if constexpr (PACKED) {
+  if constexpr (PACKED && MODE != kMerge) {
     // Tile 0 of each pair writes the rows no packed row covers: the pair's
     // heads past pack_heads and, for KV head 0, the heads whose head-map
     // entry is outside [0, Hk): NaN, padding positions zero, as the
     // per-head layout writes them.
-    if (qt == 0) {
+    if (qt == 0 && piece == 0) {
       const int extra = max(s_pk_n[0] - pk_count, 0);
       const int nh = extra + s_pk_n[1];
       const f16 qnan = (f16)__builtin_nanf("");
@@ -1385,6 +1473,12 @@ static bool use_packed_rows(const AttnParams& p) {
   return p.pack_heads >= 2 && p.M < kBM && p.Hq <= kMaxPackHeads && p.Hk > 0;
 }
 
+struct PrefillPlan {
+  PrefillGrid g;
+  bool packed;
+  size_t o_bytes, ws_bytes;  // of a split: partial O, and with (max, sum)
+};
+
 // The work list of prefill_b32_kernel (see PrefillGrid): ntq tiles per pair,
 // `group` q heads per pair, `ngroups` pairs per sequence, `total` items.
 static PrefillGrid prefill_grid(const AttnParams& p, int D, int ntq, int group, int ngroups,
@@ -1421,6 +1515,55 @@ static PrefillGrid prefill_grid(const AttnParams& p, int D, int ntq, int group, 
   g.d_band = make_fastdiv(g.band);
   g.d_gsz = make_fastdiv(g.gsz);
   return g;
+}
+
+// The tile-DMA kernel's grid, and how its items' keys are split: as many pieces
+// per item as fill the device's slots in one round, if that is at least two.
+// The lengths are known on the device only, which also caps the pieces by an
+// item's tiles; the capacity caps them here. Below kSplitFrom tiles the merge
+// launch costs more than the shorter loop gives: 8 heads x 2048 keys (64
+// tiles) 34.5 -> 33.2 us split, 32 heads x 1024 keys (32 tiles) 28.3 -> 33.3 us.
+static PrefillPlan plan_prefill(const AttnParams& p, int D) {
+  PrefillPlan plan;
+  plan.packed = use_packed_rows(p);
+  if (plan.packed) {
+    // (head, position) rows of each KV head packed into 128-row tiles
+    const int ntp = (int)(((int64_t)p.pack_heads * p.M + kBM - 1) / kBM);
+    plan.g = prefill_grid(p, D, ntp, 1, p.Hk, ntp * p.Hk * p.B, true);
+    plan.g.slots = plan.g.total;
+  } else {
+    const int ntq = (p.M + kBM - 1) / kBM;
+    const int group = (p.Hk > 0 && p.Hq % p.Hk == 0) ? p.Hq / p.Hk : 1;
+    plan.g = prefill_grid(p, D, ntq, group, p.Hq / group, ntq * p.Hq * p.B, false);
+    plan.g.slots = 8 * plan.g.per_xcd;
+  }
+  const int cap = (int)(((int64_t)p.N + 31) / 32);  // key tiles of an item at most
+  plan.g.pieces = cap < kSplitFrom ? 1
+                                   : std::max(1, std::min(kSlots / std::max(1, plan.g.slots),
+                                                          cap / kSplitMinTiles));
+  plan.g.d_slots = make_fastdiv(plan.g.slots);
+  plan.o_bytes = plan.ws_bytes = 0;
+  if (plan.g.pieces > 1) {
+    const size_t states = (size_t)plan.g.slots * plan.g.pieces;
+    plan.o_bytes = states * kBM * D * sizeof(float);
+    plan.ws_bytes = plan.o_bytes + states * kThreads * 2 * sizeof(float);
+  }
+  return plan;
+}
+
+template <int D, bool PACKED>
+static hipError_t launch_b32(AttnParams p, const PrefillPlan& plan, hipStream_t stream) {
+  const dim3 slots((unsigned)plan.g.slots), block(kThreads);
+  if (plan.g.pieces > 1 && p.ws != nullptr && p.ws_bytes >= plan.ws_bytes) {
+    p.ws_o = reinterpret_cast<float*>(p.ws);
+    p.ws_ml = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws) + plan.o_bytes);
+    const dim3 all((unsigned)(plan.g.slots * plan.g.pieces));
+    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kSplit>), all, block, 0, stream, p, plan.g);
+    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kMerge>), slots, block, 0, stream, p, plan.g);
+  } else {
+    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kWhole>), slots, block, 0, stream, p, plan.g);
+  }
+  return hipGetLastError();
 }
 
 hipError_t launch_prefill(const AttnParams& p, int D, int dtype, hipStream_t stream) {
@@ -1466,25 +1609,10 @@ hipError_t launch_prefill(const AttnParams& p, int D, int dtype, hipStream_t str
       hipLaunchKernelGGL(prefill_f16_kernel<64>, grid, dim3(kThreads), 0, stream, p);
     return hipGetLastError();
   }
-  if (use_packed_rows(p)) {
-    // (head, position) rows of each KV head packed into 128-row tiles
-    const int ntp = (int)(((int64_t)p.pack_heads * p.M + kBM - 1) / kBM);
-    const PrefillGrid g = prefill_grid(p, D, ntp, 1, p.Hk, ntp * p.Hk * p.B, true);
-    const dim3 grid((unsigned)g.total);
-    if (D == 128)
-      hipLaunchKernelGGL((prefill_b32_kernel<128, true>), grid, dim3(kThreads), 0, stream, p, g);
-    else
-      hipLaunchKernelGGL((prefill_b32_kernel<64, true>), grid, dim3(kThreads), 0, stream, p, g);
-    return hipGetLastError();
-  }
-  const int group = (p.Hk > 0 && p.Hq % p.Hk == 0) ? p.Hq / p.Hk : 1;
-  const PrefillGrid g = prefill_grid(p, D, ntq, group, p.Hq / group, ntq * p.Hq * p.B, false);
-  const dim3 grid((unsigned)(8 * g.per_xcd));
+  const PrefillPlan plan = plan_prefill(p, D);
   if (D == 128)
-    hipLaunchKernelGGL((prefill_b32_kernel<128, false>), grid, dim3(kThreads), 0, stream, p, g);
-  else
-    hipLaunchKernelGGL((prefill_b32_kernel<64, false>), grid, dim3(kThreads), 0, stream, p, g);
-  return hipGetLastError();
+    return plan.packed ? launch_b32<128, true>(p, plan, stream) : launch_b32<128, false>(p, plan, stream);
+  return plan.packed ? launch_b32<64, true>(p, plan, stream) : launch_b32<64, false>(p, plan, stream);
 }
 
 }  // namespace fa

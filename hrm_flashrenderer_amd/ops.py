@@ -173,6 +173,18 @@ def _resolve_heads_per_kv(given: Optional[int], head_map: torch.Tensor, Hk: int)
     return n
 
 
+def _prefill_split_bytes(B: int, Hq: int, Hk: int, M: int, D: int, keys: int, hpk: int) -> int:
+    """Workspace that lets the prefill kernel split the keys of a small grid
+    (FA_PREFILL_SPLIT_BYTES in the C header): at most 384 tiles of 128 query
+    rows, and at least 1505 keys (or capacity) per sequence. 0 for other calls;
+    more than the kernel uses does no harm."""
+    if keys < 1505 or Hk <= 0:
+        return 0
+    packed = 2 <= hpk and M < 128
+    tiles = B * (Hk * -(-min(hpk, Hq) * M // 128) if packed else Hq * -(-M // 128))
+    return 768 * 128 * (D + 4) * 4 if 0 < tiles <= 384 else 0
+
+
 # --------------------------------------------------------------------------
 # custom ops (bodies call the C ABI; fake impls make them traceable)
 # --------------------------------------------------------------------------
@@ -189,6 +201,8 @@ def _flash_attn_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bo
     # few query rows per K/V head (decode over a contiguous cache) take the
     # split-K decode kernels, which need a workspace
     ws_bytes = lib.fa_flash_attn_workspace_bytes(dtype, B, Hq, Hk, M, N, D)
+    if ws_bytes == 0 and dtype == _lib.FA_DTYPE_F16 and Hk > 0:
+        ws_bytes = _prefill_split_bytes(B, Hq, Hk, M, D, N, Hq // Hk)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     with _DeviceScope(q) as stream:
         _lib.check(lib.fa_flash_attn_fwd_ws(
@@ -219,6 +233,8 @@ def _flash_attn_paged_op(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.
     max_blocks = int(block_table.size(1)) if block_table is not None else 0
     cap_pages = max_blocks if block_table is not None else P
     ws_bytes = lib.fa_paged_workspace_bytes(B, Hq, M, D, Hk, cap_pages, page_size, heads_per_kv)
+    if ws_bytes == 0:
+        ws_bytes = _prefill_split_bytes(B, Hq, Hk, M, D, cap_pages * page_size, heads_per_kv)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     with _DeviceScope(q) as stream:
         args = (q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), seqlen.data_ptr(),
@@ -282,6 +298,8 @@ def _flash_attn_paged_append_op(q: torch.Tensor, k_pages: torch.Tensor, v_pages:
     max_blocks = int(block_table.size(1)) if block_table is not None else 0
     cap_pages = max_blocks if block_table is not None else P
     ws_bytes = lib.fa_paged_workspace_bytes(B, Hq, M, D, Hk, cap_pages, page_size, heads_per_kv)
+    if ws_bytes == 0:
+        ws_bytes = _prefill_split_bytes(B, Hq, Hk, M, D, cap_pages * page_size, heads_per_kv)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     with _DeviceScope(q) as stream:
         _lib.check(lib.fa_flash_attn_paged_append_fwd(

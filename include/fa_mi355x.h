@@ -49,6 +49,17 @@ extern "C" {
 #define FA_ERR_WORKSPACE -3 /* workspace missing or smaller than needed */
 
 /*
+ * Optional workspace of the fp16 prefill kernel. A call off the decode kernels
+ * needs no workspace (its fa_*_workspace_bytes is 0). When its grid is small
+ * for its keys (at most 384 tiles of 128 query rows, at least 1505 keys per
+ * sequence: one request's prompt chunk over a long context), a workspace of
+ * this many bytes lets the kernel split the keys over idle compute units and
+ * merge the parts in a second launch; with less it runs unsplit. The two agree
+ * within fp32 rounding of the softmax sums, not bit for bit.
+ */
+#define FA_PREFILL_SPLIT_BYTES(D) ((size_t)768 * 128 * ((size_t)(D) + 4) * 4)
+
+/*
  * Contiguous attention: O = softmax(Q K^T / sqrt(D) + causal mask) V.
  * Replaces _ext.flash_attn_fwd (csrc/ext.cpp:30-40) and its launcher
  * flash_attn_fwd_cuda (csrc/flash_attn_sm75.cu:428-467).
@@ -76,7 +87,8 @@ int fa_flash_attn_fwd(const void* q, const void* k, const void* v, void* o,
  * single-token decode over a contiguous cache) split each K/V head's keys
  * over the whole device and merge the partial results in a second kernel,
  * while other calls take the prefill kernels exactly as fa_flash_attn_fwd
- * does. Arguments and results are fa_flash_attn_fwd's.
+ * does, unless the workspace has FA_PREFILL_SPLIT_BYTES. Arguments and results
+ * are fa_flash_attn_fwd's.
  *   workspace : device scratch of at least fa_flash_attn_workspace_bytes(...)
  *               bytes for the same sizes (may be NULL when that is 0); its
  *               contents need no initialisation.
