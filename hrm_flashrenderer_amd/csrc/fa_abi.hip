@@ -317,7 +317,20 @@ static int paged_fwd(const void* q, const void* k_pages, const void* v_pages,
   p.rope_len = rope_len;
 
   (void)hipGetLastError();
-  const bool decode = decode_ok && fa::use_decode_path(B, M, Hq, Hk, heads_per_kv);
+  // Calls of the decode path (by its shapes, and so by its workspace) with more
+  // rows per KV head than one pass of the decode kernels run on the packed
+  // prefill tiles, their keys split in that workspace.
+  const bool decode_shape = decode_ok && fa::use_decode_path(B, M, Hq, Hk, heads_per_kv);
+  const bool decode = decode_shape && !fa::packed_beats_decode(M, Hq, heads_per_kv, PS);
+  size_t decode_bytes = 0;
+  if (decode_shape && (int64_t)B * Hq * M > 0) {
+    // plan_decode sizes the workspace for one launch of at most
+    // kDecodeMaxBatch sequences
+    decode_bytes = fa::plan_decode(B, Hq, M, D, Hk, p.N, heads_per_kv).ws_bytes;
+    if (workspace == nullptr || workspace_bytes < decode_bytes)
+      return fail(FA_ERR_WORKSPACE, "workspace of %zu bytes required, got %zu", decode_bytes,
+                  workspace == nullptr ? (size_t)0 : workspace_bytes);
+  }
   if (app != nullptr) {
     p.app_advance = app->advance ? 1 : 0;
     // the decode kernels take the token in advance mode, where it is every
@@ -353,14 +366,10 @@ static int paged_fwd(const void* q, const void* k_pages, const void* v_pages,
                                   p.rope_cos, p.rope_sin, rope_len, (hipStream_t)stream);
     }
   } else if (decode) {
-    // plan_decode sizes the workspace for one launch of at most
-    // kDecodeMaxBatch sequences; a larger batch runs in such launches one
-    // after another on the stream, each on the workspace the previous one
-    // has finished with (its combine kernel runs before the next launch).
+    // a batch beyond kDecodeMaxBatch runs in such launches one after another
+    // on the stream, each on the workspace the previous one has finished with
+    // (its combine kernel runs before the next launch)
     const fa::DecodePlan plan = fa::plan_decode(B, Hq, M, D, Hk, p.N, heads_per_kv);
-    if (workspace == nullptr || workspace_bytes < plan.ws_bytes)
-      return fail(FA_ERR_WORKSPACE, "workspace of %zu bytes required, got %zu", plan.ws_bytes,
-                  workspace == nullptr ? (size_t)0 : workspace_bytes);
     char* ws = reinterpret_cast<char*>(workspace);
     for (int b0 = 0; b0 < B && e == hipSuccess; b0 += fa::kDecodeMaxBatch) {
       const int Bc = std::min(fa::kDecodeMaxBatch, B - b0);
@@ -404,7 +413,8 @@ static int paged_fwd(const void* q, const void* k_pages, const void* v_pages,
     // heads_per_kv of them) into shared 128-row tiles when M < 128
     p.pack_heads = heads_per_kv > 0 ? std::min(heads_per_kv, Hq) : 0;
     p.ws = workspace;
-    p.ws_bytes = workspace_bytes;
+    // the same split whatever the caller's workspace has beyond what it must
+    p.ws_bytes = decode_shape ? decode_bytes : workspace_bytes;
     e = fa::launch_prefill(p, D, FA_DTYPE_F16, (hipStream_t)stream);
   }
   // the decode path's combine kernel advances the lengths itself (from the

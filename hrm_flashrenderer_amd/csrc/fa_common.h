@@ -170,7 +170,7 @@ struct AttnParams {
   const f16* app_v;
   int app_advance;               // 0 or 1
   int* ws_app;                   // [B] positions the decode kernel publishes to the combine kernel
-  // prefill: the caller's workspace (nullable), for a split of the keys
+  // prefill: the workspace (nullable) that a split of the keys may use
   void* ws;
   size_t ws_bytes;
 
@@ -284,6 +284,9 @@ hipError_t launch_paged_append(void* k_pages, void* v_pages, const void* k_new, 
                                const f16* rope_cos, const f16* rope_sin, int rope_len,
                                hipStream_t stream);
 hipError_t launch_prefill(const AttnParams& p, int D, int dtype, hipStream_t stream);
+// Whether a paged call of the decode path runs on the packed prefill tiles
+// instead, with the decode path's workspace for their split.
+bool packed_beats_decode(int M, int Hq, int heads_per_kv, int PS);
 hipError_t launch_decode(const AttnParams& p, int D, hipStream_t stream);
 
 // Sequences of one decode launch: a larger batch runs in launches of at most

@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(AttnParams p) {
 // two LDS stages of its own (2 x 16 KB at D = 128, no barrier in the loop) and
 // runs the prefill kernel's tile: S^T = K Q^T and O^T = V^T P^T on
 // 32x32x16 MFMAs, the V operand by the transposing LDS read, both operands
-// read once for the NB blocks of 32 rows. K's stage is refilled once QK^T has
+// read once for the NB (1 or 2) blocks of 32 rows. K's stage is refilled once QK^T has
 // read it and V's after PV, so 16 to 32 KB per wave are in flight. The tile
 // then costs about a third of the time its bytes take at the streaming rate
 // (NB = 2).
@@ -860,10 +860,9 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
   constexpr int NSLAB = BN / SL;
   constexpr int IPS = SL / C::RPI;          // DMA instructions per slab
   constexpr int NDMA = NSLAB * IPS;         // per tile of K (and of V)
-  constexpr int NM = NB < 2 ? NB : 2;       // blocks merged at a time: they fill the stages
   constexpr int CF = D / 4;                 // 16-byte chunks of a partial fp32 row
   static_assert(IPS >= 1, "slab smaller than one wave-wide load");
-  static_assert(NM * 32 * D * 4 <= 4 * TILE, "merge buffer larger than a wave's stages");
+  static_assert(NB * 32 * D * 4 <= 4 * TILE, "merge buffer larger than a wave's stages");
   // a store address the caller's workspace only aligns to 4 bytes
   typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -967,7 +966,6 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
 
     for (int rc0 = 0; rc0 < nrows; rc0 += 32 * NB) {
       if (rc0 > 0) dma_tile(0, 0);  // a later pass over the same groups
-      bool blk_live[NB];
       int row_lim[NB];          // keys j < row_lim are visible to this lane's row
       half8 qreg[NB][KSTEPS];
       float m_ref[NB], neg_m[NB], thr[NB], l_run[NB];
@@ -975,7 +973,6 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
 #pragma unroll
       for (int bk = 0; bk < NB; ++bk) {
         const int rc = rc0 + 32 * bk;
-        blk_live[bk] = rc < nrows;
         const bool row_ok = rc + col < nrows;
         const int ridx = row_ok ? rc + col : 0;
         const int hi = ridx / p.M;
@@ -1047,7 +1044,6 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
         half8 pb[NB][2];
 #pragma unroll
         for (int bk = 0; bk < NB; ++bk) {
-          if (NB > 2 && !blk_live[bk]) continue;
           if (k0 + BN > min_lim) {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
@@ -1084,8 +1080,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
           const int st = m / DBLK, i = m % DBLK;
 #pragma unroll
           for (int bk = 0; bk < NB; ++bk) {
-            if (NB <= 2 || blk_live[bk])
-              acc[bk][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[m % VA], pb[bk][st], acc[bk][i], 0, 0, 0);
+            acc[bk][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[m % VA], pb[bk][st], acc[bk][i], 0, 0, 0);
           }
           if (m + VA < NMF) va[m % VA] = ld_vt<D>(buf, vofs, (m + VA) / DBLK, (m + VA) % DBLK);
         }
@@ -1099,9 +1094,9 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
       // the DMAs past the last tile write zeros to the stages reused below
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-      // Merge of the four waves' states, NM blocks at a time: each wave
-      // leaves rows of D floats (16-byte chunks swizzled by the row) in its
-      // own stages, then every thread sums 16-byte pieces over the waves.
+      // Merge of the four waves' states: each wave leaves rows of D floats
+      // (16-byte chunks swizzled by the row) in its own stages, then every
+      // thread sums 16-byte pieces over the waves.
 #pragma unroll
       for (int bk = 0; bk < NB; ++bk) {
         const float l_tot = l_run[bk] + __shfl_xor(l_run[bk], 32);
@@ -1109,50 +1104,41 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
           s_m[wave][32 * bk + col] = m_ref[bk];
           s_l[wave][32 * bk + col] = l_tot;
         }
-      }
 #pragma unroll
-      for (int b0 = 0; b0 < NB; b0 += NM) {
-        if (rc0 + 32 * b0 >= nrows) break;
-        if (b0 > 0) __syncthreads();  // the previous blocks have been read
+        for (int i = 0; i < DBLK; ++i) {
 #pragma unroll
-        for (int j = 0; j < NM; ++j) {
-#pragma unroll
-          for (int i = 0; i < DBLK; ++i) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const floatx16& a = acc[b0 + j][i];
-              *reinterpret_cast<floatx4*>(stage + (32 * j + col) * 4 * D +
-                                          16 * ((8 * i + 2 * g + half_id) ^ (col % CF))) =
-                  floatx4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
-            }
+          for (int g = 0; g < 4; ++g) {
+            const floatx16& a = acc[bk][i];
+            *reinterpret_cast<floatx4*>(stage + (32 * bk + col) * 4 * D +
+                                        16 * ((8 * i + 2 * g + half_id) ^ (col % CF))) =
+                floatx4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
           }
         }
-        __syncthreads();
-        for (int e = tid; e < NM * 32 * CF; e += kDecodeThreads) {
-          const int row = e / CF, ch = e % CF;
-          const int lr = 32 * b0 + row;      // row of the pass
-          const int ri = rc0 + lr;           // row of the slot
-          if (ri >= nrows || ri >= p.dec_rows) continue;  // rows past the slot: NaN in the combine
-          float mx = s_m[0][lr];
+      }
+      __syncthreads();
+      for (int e = tid; e < NB * 32 * CF; e += kDecodeThreads) {
+        const int row = e / CF, ch = e % CF;
+        const int ri = rc0 + row;          // row of the slot
+        if (ri >= nrows || ri >= p.dec_rows) break;  // rows past the slot: NaN in the combine
+        float mx = s_m[0][row];
 #pragma unroll
-          for (int w = 1; w < kDecodeWaves; ++w) mx = fmaxf(mx, s_m[w][lr]);
-          float lsum = 0.f;
-          floatx4 osum = floatx4{0.f, 0.f, 0.f, 0.f};
-          if (mx != -INFINITY) {
+        for (int w = 1; w < kDecodeWaves; ++w) mx = fmaxf(mx, s_m[w][row]);
+        float lsum = 0.f;
+        floatx4 osum = floatx4{0.f, 0.f, 0.f, 0.f};
+        if (mx != -INFINITY) {
 #pragma unroll
-            for (int w = 0; w < kDecodeWaves; ++w) {
-              const float a = __builtin_amdgcn_exp2f(s_m[w][lr] - mx);
-              lsum += a * s_l[w][lr];
-              osum += a * *reinterpret_cast<const floatx4*>(smem + w * 4 * TILE + row * 4 * D +
-                                                            16 * (ch ^ (row % CF)));
-            }
+          for (int w = 0; w < kDecodeWaves; ++w) {
+            const float a = __builtin_amdgcn_exp2f(s_m[w][row] - mx);
+            lsum += a * s_l[w][row];
+            osum += a * *reinterpret_cast<const floatx4*>(smem + w * 4 * TILE + row * 4 * D +
+                                                          16 * (ch ^ (row % CF)));
           }
-          const int64_t srow = (int64_t)slot * p.dec_rows + ri;
-          *reinterpret_cast<floatx4u*>(p.ws_o + srow * D + 4 * ch) = osum;
-          if (ch == 0) {
-            p.ws_ml[srow * 2 + 0] = mx;
-            p.ws_ml[srow * 2 + 1] = lsum;
-          }
+        }
+        const int64_t srow = (int64_t)slot * p.dec_rows + ri;
+        *reinterpret_cast<floatx4u*>(p.ws_o + srow * D + 4 * ch) = osum;
+        if (ch == 0) {
+          p.ws_ml[srow * 2 + 0] = mx;
+          p.ws_ml[srow * 2 + 1] = lsum;
         }
       }
       __syncthreads();  // the stages, s_m and s_l are free again
@@ -1374,8 +1360,10 @@ __global__ __launch_bounds__(WIDE ? 64 * kWideWaves : 256) void decode_combine_k
 }
 
 // The decode kernel variant a call runs.
-//  * wide_nb > 0: decode_wide_kernel with that many 32-row blocks per pass and
-//    slabs of wide_sl keys (decode_is_wide).
+//  * wide_nb > 0: decode_wide_kernel with that many 32-row blocks per pass (at
+//    most 2: four spill at D = 128, and more than 64 rows run on the packed
+//    prefill tiles where heads_per_kv is known) and slabs of wide_sl keys
+//    (decode_is_wide).
 //  * else decode_kernel: row loads from whole 16-token groups (aligned: pages
 //    of a multiple of 16 tokens, or unpaged rows at a fixed stride whose
 //    16-row span fits a buffer range) or one by one, the fp32-query split
@@ -1393,8 +1381,6 @@ struct DecodeVariant {
 };
 
 constexpr int max_row_blocks(int D) { return D == 128 ? 2 : 4; }
-// four 32-row blocks spill at D = 128
-constexpr int max_wide_blocks(int D) { return D == 128 ? 2 : 4; }
 
 // Whether the 32-key LDS tiles serve a call with `rows` query rows per KV head:
 // contiguous K/V or pages of whole 8-key slabs, and either more rows than one
@@ -1410,7 +1396,7 @@ DecodeVariant decode_variant(const AttnParams& p) {
   v.append = p.app_k != nullptr;
   if (!v.qsplit && !v.append && (p.kv.paged || p.kv.stride_tok == p.kv.D) &&
       decode_is_wide(p.kv.paged, p.kv.PS, p.dec_rows)) {
-    v.wide_nb = p.dec_rows <= 32 ? 1 : p.dec_rows <= 64 ? 2 : max_wide_blocks(p.kv.D);
+    v.wide_nb = p.dec_rows <= 32 ? 1 : 2;
     v.wide_sl = p.kv.paged && p.kv.PS % 16 != 0 ? 8 : 16;
     return v;
   }
@@ -1428,8 +1414,7 @@ DecodeVariant decode_variant(const AttnParams& p) {
 template <int D, int SL>
 const void* decode_wide_fn(int nb) {
   return nb == 1 ? reinterpret_cast<const void*>(&decode_wide_kernel<D, 1, SL>)
-       : nb == 2 ? reinterpret_cast<const void*>(&decode_wide_kernel<D, 2, SL>)
-                 : reinterpret_cast<const void*>(&decode_wide_kernel<D, max_wide_blocks(D), SL>);
+                 : reinterpret_cast<const void*>(&decode_wide_kernel<D, 2, SL>);
 }
 
 template <int D>
@@ -1493,13 +1478,14 @@ bool use_decode_path(int B, int M, int Hq, int Hk, int heads_per_kv) {
   if (rows <= 2 * kRows) return true;
   // With M < 128 and a heads_per_kv bound, the prefill kernel packs a KV
   // head's (head, position) rows into 128-row tiles: one pass over its pages
-  // for all of them at prefill MFMA rates. That wins once the tiles fill the
-  // device; with fewer, the decode kernels (split over the whole device)
-  // serve the rows in passes of up to 64. Over cfg4's pool at 64/8 heads,
-  // M = 16 (two decode passes): B = 1 82 us decode against 293 packed, B = 16
-  // 358 against 361, B = 32 (256 tiles) packed 396, B = 64 559 against 1281;
-  // M = 8 (one decode pass, half-empty tiles): B = 32 350 decode against 389
-  // packed, B = 64 (512 tiles) 512 packed against 651.
+  // for all of them at prefill MFMA rates. That needs no workspace once the
+  // tiles fill the device; with fewer, the call is sized as a decode call: up
+  // to 64 rows it runs on the decode kernels (split over the whole device), and
+  // with more on the packed tiles with their keys split in that workspace
+  // (packed_beats_decode). With up to 64 rows the tiles are half empty, so the
+  // line lies at twice as many: M = 8, 64/8 heads, 1024-16384 keys, 64
+  // sequences (512 tiles) 512 us packed against 651 on one decode pass, 32
+  // sequences 389 against 350.
   const bool packable = heads_per_kv >= 2 && M < 128;
   if (packable) {
     const int64_t hpk = std::min(heads_per_kv, Hq);

@@ -1464,6 +1464,18 @@ __global__ __launch_bounds__(64 * kF32Waves) void prefill_f32_kernel(AttnParams 
 
 }  // namespace
 
+// More rows per KV head than one pass of decode_wide_kernel (64 at D = 128):
+// the packed tiles take up to 128 in one pass, and their split keys fill the
+// device where the tiles alone do not. 64/8 heads, D = 128, decode passes ->
+// packed: M = 16, 16 sequences of 1024-8192 keys 155 -> 92 us, one sequence of
+// 16000 keys 60 -> 46 us, of 300 keys 48 -> 26 us; M = 9, 1000 keys 31 -> 26 us.
+// Up to 64 rows the decode pass is the faster one over long contexts (M = 5,
+// one sequence of 16000 keys: 33 us against 44).
+bool packed_beats_decode(int M, int Hq, int heads_per_kv, int PS) {
+  const int64_t hpk = std::min(heads_per_kv, Hq);
+  return PS % 8 == 0 && hpk >= 2 && M < kBM && Hq <= kMaxPackHeads && hpk * M > 64;
+}
+
 // The packed layout serves calls with fewer than 128 rows per q head and at
 // least two q heads per KV head (pack_heads, from the caller's heads_per_kv),
 // on the tile-DMA kernel: it fills 128-row tiles with the (head, position)
@@ -1476,7 +1488,7 @@ static bool use_packed_rows(const AttnParams& p) {
 struct PrefillPlan {
   PrefillGrid g;
   bool packed;
-  size_t o_bytes, ws_bytes;  // of a split: partial O, and with (max, sum)
+  size_t o_bytes;  // of a split: partial O, before the (max, sum)s
 };
 
 // The work list of prefill_b32_kernel (see PrefillGrid): ntq tiles per pair,
@@ -1542,19 +1554,19 @@ static PrefillPlan plan_prefill(const AttnParams& p, int D) {
                                    : std::max(1, std::min(kSlots / std::max(1, plan.g.slots),
                                                           cap / kSplitMinTiles));
   plan.g.d_slots = make_fastdiv(plan.g.slots);
-  plan.o_bytes = plan.ws_bytes = 0;
-  if (plan.g.pieces > 1) {
-    const size_t states = (size_t)plan.g.slots * plan.g.pieces;
-    plan.o_bytes = states * kBM * D * sizeof(float);
-    plan.ws_bytes = plan.o_bytes + states * kThreads * 2 * sizeof(float);
-  }
+  // ... and by the states that the workspace holds
+  const size_t state_o = (size_t)kBM * D * sizeof(float);
+  const size_t state = state_o + kThreads * 2 * sizeof(float);
+  const size_t held = p.ws == nullptr ? 0 : p.ws_bytes / state / std::max(1, plan.g.slots);
+  plan.g.pieces = held < 2 ? 1 : (int)std::min<size_t>(plan.g.pieces, held);
+  plan.o_bytes = state_o * plan.g.slots * plan.g.pieces;
   return plan;
 }
 
 template <int D, bool PACKED>
 static hipError_t launch_b32(AttnParams p, const PrefillPlan& plan, hipStream_t stream) {
   const dim3 slots((unsigned)plan.g.slots), block(kThreads);
-  if (plan.g.pieces > 1 && p.ws != nullptr && p.ws_bytes >= plan.ws_bytes) {
+  if (plan.g.pieces > 1) {
     p.ws_o = reinterpret_cast<float*>(p.ws);
     p.ws_ml = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws) + plan.o_bytes);
     const dim3 all((unsigned)(plan.g.slots * plan.g.pieces));

@@ -54,8 +54,9 @@ extern "C" {
  * for its keys (at most 384 tiles of 128 query rows, at least 1505 keys per
  * sequence: one request's prompt chunk over a long context), a workspace of
  * this many bytes lets the kernel split the keys over idle compute units and
- * merge the parts in a second launch; with less it runs unsplit. The two agree
- * within fp32 rounding of the softmax sums, not bit for bit.
+ * merge the parts in a second launch; with less it makes fewer parts or runs
+ * unsplit. The results agree within fp32 rounding of the softmax sums, not bit
+ * for bit.
  */
 #define FA_PREFILL_SPLIT_BYTES(D) ((size_t)768 * 128 * ((size_t)(D) + 4) * 4)
 

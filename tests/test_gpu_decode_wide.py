@@ -1,6 +1,7 @@
 """Decode on 32-key LDS tiles (more than 16 query rows per KV head, or pages of
 8, 24, ... tokens): every row-block count at its edges (16/17, 32/33, 64/65 rows
-and a second pass), slabs of 16 and of 8 keys, pages with and without a table,
+and a second pass, which calls without a heads_per_kv bound take; with one,
+more than 64 rows run on packed prefill tiles in the decode workspace), slabs of 16 and of 8 keys, pages with and without a table,
 contiguous K/V, rows that see only part of the keys, padding rows, rotary
 queries and lengths that end inside a slab or leave waves without a tile,
 against the fp64 oracle; dead slots hold NaN. The one-call decode step equals
@@ -46,6 +47,7 @@ def _paged(gpu, Hk, D, PS, lengths, table, seed):
     (10, 2, 1, 64, 24, False, False),
     (20, 2, 4, 128, 24, True, True),     # 40 rows
     (12, 1, 8, 64, 8, True, True),       # 96 rows
+    (71, 1, 1, 128, 16, True, False),    # 71 rows of one token
 ])
 def test_wide_decode(gpu, Hq, Hk, M, D, PS, table, causal):
     lengths = [1, 40, 777, 0, 128, 2049]
@@ -58,9 +60,12 @@ def test_wide_decode(gpu, Hq, Hk, M, D, PS, table, causal):
     qo = torch.tensor(offs, dtype=torch.int32, device=gpu) if causal else 0
     tab = bt.to(gpu) if table else None
     out = flash_attn_paged(q, k, v, seqlen, PS, hm, causal, qo, block_table=tab)
+    unbound = torch.ops.hrm_fa.flash_attn_paged(
+        q, k, v, seqlen, PS, hm, causal, 0, 0, qo if causal else None, None, tab, None, None, None, 0)
     ref = paged_reference(q, k, v, bt, lengths, PS, hm, causal, offs)
     for (b, h), r in ref.items():
         assert_close(out[b, h].cpu().numpy(), r, f"b={b} h={h}")
+        assert_close(unbound[b, h].cpu().numpy(), r, f"no bound b={b} h={h}")
     # padding rows come out as zeros and leave the others alone
     lens = torch.tensor([M, max(0, M - 2), M, M, 1, M], dtype=torch.int32, device=gpu)
     part = flash_attn_paged(q, k, v, seqlen, PS, hm, causal, qo, block_table=tab, q_lens=lens)
@@ -78,7 +83,7 @@ def test_wide_contiguous(gpu, Hq, Hk, M, N, D):
 
 
 @pytest.mark.parametrize("rope", [False, True])
-@pytest.mark.parametrize("Hq,Hk,D,PS", [(48, 2, 128, 16), (8, 2, 64, 8), (20, 1, 128, 24)])
+@pytest.mark.parametrize("Hq,Hk,D,PS", [(48, 2, 128, 16), (8, 2, 64, 8), (20, 1, 128, 24), (71, 1, 64, 16)])
 def test_step_equals_two_calls(gpu, Hq, Hk, D, PS, rope):
     lengths = [5, 0, 300, 127]
     B = len(lengths)
