@@ -11,8 +11,8 @@ conventions as the reference, flashattention_custom/ops.py:79-99):
 
 Each validates its arguments in Python with the reference extension's
 messages (csrc/ext.cpp:30-89), then calls a `torch.library` custom op
-(`hrm_fa::*`) whose body calls the C ABI of libfa_mi355x.so on the current
-stream of the tensors' device. There is no CPU fallback: tensors must be on a
+(`hrm_fa::*`), or for plain tensors its body at once (`_direct`), which calls
+the C ABI of libfa_mi355x.so on the current stream of the tensors' device. There is no CPU fallback: tensors must be on a
 ROCm device and the library must be built, otherwise a RuntimeError is raised
 (the reference's `_ext` raises the same "CUDA required" checks; the wording
 refers to torch's device type, which is "cuda" on ROCm).
@@ -38,6 +38,8 @@ import weakref
 from typing import Optional, Union
 
 import torch
+from torch.autograd import forward_ad
+from torch.autograd.graph import increment_version
 
 from . import _lib
 
@@ -69,7 +71,7 @@ class _DeviceScope:
         if cur != self.idx:
             self.prev = cur
             torch.cuda.set_device(self.idx)
-        return torch.cuda.current_stream(self.idx).cuda_stream
+        return torch._C._cuda_getCurrentRawStream(self.idx)
 
     def __exit__(self, *exc):
         if self.prev is not None:
@@ -121,6 +123,35 @@ def _check_rope(rope, D: int, device: torch.device, require_device: bool = True)
            "rope tables cos/sin [L, D/2] required")
     _check(cos.device == device and sin.device == device, "tensors must be on one device")
     return cos, sin
+
+
+def _direct(*tensors: Optional[torch.Tensor]) -> bool:
+    """Whether a call may run the body of its custom op without the dispatcher,
+    which costs 6-9 us of host time per call (flash_attn 18.5 -> 12 us, where
+    the kernels of a small call take 10). That is so for plain tensors when
+    nothing could see or change the call on its way: no tracing or
+    compilation, no dispatch, function or functorch mode, no forward-mode
+    level, no profiler, no tensor whose gradient would be recorded, no
+    subclass and no lazily negated or zero tensor."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+            or torch._C._autograd._profiler_enabled()):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) is not torch.Tensor or (grad and t.requires_grad)
+                              or t.is_neg() or t._is_zerotensor()):
+            return False
+    return True
+
+
+def _mutated(*tensors: torch.Tensor) -> None:
+    """Bump the version counters of tensors a directly run body wrote, as the
+    dispatcher does for the arguments an op mutates (inference tensors have
+    none)."""
+    increment_version([t for t in tensors if not t.is_inference()])
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -189,8 +220,7 @@ def _prefill_split_bytes(B: int, Hq: int, Hk: int, M: int, D: int, keys: int, hp
 # custom ops (bodies call the C ABI; fake impls make them traceable)
 # --------------------------------------------------------------------------
 
-@torch.library.custom_op("hrm_fa::flash_attn", mutates_args=())
-def _flash_attn_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool,
+def _flash_attn_body(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool,
                    q_offset: int, k_offset: int, q_offsets: Optional[torch.Tensor],
                    k_offsets: Optional[torch.Tensor]) -> torch.Tensor:
     lib = _lib.load()
@@ -212,13 +242,15 @@ def _flash_attn_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bo
     return o
 
 
+_flash_attn_op = torch.library.custom_op("hrm_fa::flash_attn", mutates_args=())(_flash_attn_body)
+
+
 @_flash_attn_op.register_fake
 def _(q, k, v, causal, q_offset, k_offset, q_offsets, k_offsets):
     return torch.empty_like(q)
 
 
-@torch.library.custom_op("hrm_fa::flash_attn_paged", mutates_args=())
-def _flash_attn_paged_op(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
+def _flash_attn_paged_body(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                          seqlen: torch.Tensor, page_size: int, head_map: torch.Tensor,
                          causal: bool, q_offset: int, k_offset: int,
                          q_offsets: Optional[torch.Tensor], k_offsets: Optional[torch.Tensor],
@@ -249,14 +281,16 @@ def _flash_attn_paged_op(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.
     return o
 
 
+_flash_attn_paged_op = torch.library.custom_op("hrm_fa::flash_attn_paged", mutates_args=())(_flash_attn_paged_body)
+
+
 @_flash_attn_paged_op.register_fake
 def _(q, k_pages, v_pages, seqlen, page_size, head_map, causal, q_offset, k_offset, q_offsets,
       k_offsets, block_table, rope_cos, rope_sin, q_lens=None, heads_per_kv=0):
     return torch.empty_like(q)
 
 
-@torch.library.custom_op("hrm_fa::paged_kv_append", mutates_args=("k_pages", "v_pages"))
-def _paged_kv_append_op(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: torch.Tensor,
+def _paged_kv_append_body(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: torch.Tensor,
                         v_new: torch.Tensor, start_pos: int, start_positions: Optional[torch.Tensor],
                         page_size: int, block_table: Optional[torch.Tensor],
                         rope_cos: Optional[torch.Tensor], rope_sin: Optional[torch.Tensor]) -> None:
@@ -275,15 +309,16 @@ def _paged_kv_append_op(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: tor
                 *args, rope_cos.data_ptr(), rope_sin.data_ptr(), rope_cos.size(0), stream))
 
 
+_paged_kv_append_op = torch.library.custom_op("hrm_fa::paged_kv_append", mutates_args=("k_pages", "v_pages"))(_paged_kv_append_body)
+
+
 @_paged_kv_append_op.register_fake
 def _(k_pages, v_pages, k_new, v_new, start_pos, start_positions, page_size, block_table,
       rope_cos, rope_sin):
     return None
 
 
-@torch.library.custom_op("hrm_fa::flash_attn_paged_append",
-                         mutates_args=("k_pages", "v_pages", "seqlen"))
-def _flash_attn_paged_append_op(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
+def _flash_attn_paged_append_body(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                                 seqlen: torch.Tensor, page_size: int, head_map: torch.Tensor,
                                 causal: bool, q_offset: int, q_offsets: Optional[torch.Tensor],
                                 block_table: Optional[torch.Tensor], k_new: torch.Tensor,
@@ -312,14 +347,16 @@ def _flash_attn_paged_append_op(q: torch.Tensor, k_pages: torch.Tensor, v_pages:
     return o
 
 
+_flash_attn_paged_append_op = torch.library.custom_op("hrm_fa::flash_attn_paged_append", mutates_args=("k_pages", "v_pages", "seqlen"))(_flash_attn_paged_append_body)
+
+
 @_flash_attn_paged_append_op.register_fake
 def _(q, k_pages, v_pages, seqlen, page_size, head_map, causal, q_offset, q_offsets, block_table,
       k_new, v_new, advance, start_pos, start_positions, rope_cos, rope_sin, heads_per_kv=0):
     return torch.empty_like(q)
 
 
-@torch.library.custom_op("hrm_fa::paged_kv_scatter", mutates_args=("k_pages", "v_pages"))
-def _paged_kv_scatter_op(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: torch.Tensor,
+def _paged_kv_scatter_body(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: torch.Tensor,
                          v_new: torch.Tensor, positions: torch.Tensor, page_size: int,
                          block_table: Optional[torch.Tensor], rope_cos: Optional[torch.Tensor],
                          rope_sin: Optional[torch.Tensor]) -> None:
@@ -333,6 +370,9 @@ def _paged_kv_scatter_op(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: to
             B, Hk, T, D, NB, P, page_size, positions.data_ptr(), _ptr(block_table), max_blocks,
             _ptr(rope_cos), _ptr(rope_sin), rope_cos.size(0) if rope_cos is not None else 0,
             stream))
+
+
+_paged_kv_scatter_op = torch.library.custom_op("hrm_fa::paged_kv_scatter", mutates_args=("k_pages", "v_pages"))(_paged_kv_scatter_body)
 
 
 @_paged_kv_scatter_op.register_fake
@@ -384,7 +424,8 @@ def flash_attn(q, k, v, causal=True, q_offset=0, k_offset=0):
     B = q.size(0)
     qo, qo_t = _per_seq(q_offset, B, "q_offset", q.device)
     ko, ko_t = _per_seq(k_offset, B, "k_offset", q.device)
-    return _flash_attn_op(q, k, v, bool(causal), qo, ko, qo_t, ko_t)
+    run = _flash_attn_body if _direct(q, k, v, qo_t, ko_t) else _flash_attn_op
+    return run(q, k, v, bool(causal), qo, ko, qo_t, ko_t)
 
 
 def validate_flash_attn_paged(q, k_pages, v_pages, seqlen, page_size, head_map,
@@ -451,8 +492,11 @@ def flash_attn_paged(q, k_pages, v_pages, seqlen, page_size, head_map,
         _check(q_lens.is_contiguous(), "contiguous required")
         _check(q_lens.dim() == 1 and q_lens.numel() == B, "q_lens [B] required")
     hpk = _resolve_heads_per_kv(heads_per_kv, head_map, k_pages.size(1))
-    return _flash_attn_paged_op(q, k_pages, v_pages, seqlen, page_size, head_map, bool(causal),
-                                qo, ko, qo_t, ko_t, block_table, cos, sin, q_lens, hpk)
+    run = (_flash_attn_paged_body
+           if _direct(q, k_pages, v_pages, seqlen, head_map, qo_t, ko_t, block_table, cos, sin, q_lens)
+           else _flash_attn_paged_op)
+    return run(q, k_pages, v_pages, seqlen, page_size, head_map, bool(causal), qo, ko, qo_t, ko_t,
+               block_table, cos, sin, q_lens, hpk)
 
 
 def validate_paged_kv_append(k_pages, v_pages, k_new, v_new, start_pos, page_size,
@@ -509,7 +553,12 @@ def paged_kv_append(k_pages, v_pages, k_new, v_new, start_pos, page_size, *, blo
             _check(sp + k_new.size(2) <= cos.size(0),
                    f"positions {sp}..{sp + k_new.size(2) - 1} are outside the rotary table "
                    f"of {cos.size(0)}")
-    _paged_kv_append_op(k_pages, v_pages, k_new, v_new, sp, sp_t, page_size, block_table, cos, sin)
+    args = (k_pages, v_pages, k_new, v_new, sp, sp_t, page_size, block_table, cos, sin)
+    if _direct(k_pages, v_pages, k_new, v_new, sp_t, block_table, cos, sin):
+        _paged_kv_append_body(*args)
+        _mutated(k_pages, v_pages)
+    else:
+        _paged_kv_append_op(*args)
 
 
 def flash_attn_paged_append(q, k_pages, v_pages, k_new, v_new, seqlen, page_size, head_map,
@@ -564,9 +613,14 @@ def flash_attn_paged_append(q, k_pages, v_pages, k_new, v_new, seqlen, page_size
                    f"positions {qo}..{qo + q.size(2) - 1} are outside the rotary table "
                    f"of {cos.size(0)}")
     hpk = _resolve_heads_per_kv(heads_per_kv, head_map, k_pages.size(1))
-    return _flash_attn_paged_append_op(q, k_pages, v_pages, seqlen, page_size, head_map,
-                                       bool(causal), qo, qo_t, block_table, k_new, v_new,
-                                       advance, sp, sp_t, cos, sin, hpk)
+    args = (q, k_pages, v_pages, seqlen, page_size, head_map, bool(causal), qo, qo_t, block_table,
+            k_new, v_new, advance, sp, sp_t, cos, sin, hpk)
+    if not _direct(q, k_pages, v_pages, seqlen, head_map, qo_t, block_table, k_new, v_new, sp_t,
+                   cos, sin):
+        return _flash_attn_paged_append_op(*args)
+    o = _flash_attn_paged_append_body(*args)
+    _mutated(k_pages, v_pages, seqlen)
+    return o
 
 
 def paged_kv_scatter(k_pages, v_pages, k_new, v_new, positions, page_size, *, block_table=None,
@@ -595,5 +649,9 @@ def paged_kv_scatter(k_pages, v_pages, k_new, v_new, positions, page_size, *, bl
     cos, sin = _check_rope(rope, k_new.size(3), k_new.device)
     if cos is not None:
         _check(k_new.size(3) % 16 == 0, "rotary append needs head_dim a multiple of 16")
-    _paged_kv_scatter_op(k_pages, v_pages, k_new, v_new, positions, page_size, block_table,
-                         cos, sin)
+    args = (k_pages, v_pages, k_new, v_new, positions, page_size, block_table, cos, sin)
+    if _direct(k_pages, v_pages, k_new, v_new, positions, block_table, cos, sin):
+        _paged_kv_scatter_body(*args)
+        _mutated(k_pages, v_pages)
+    else:
+        _paged_kv_scatter_op(*args)
