@@ -308,11 +308,18 @@ DecodePlan plan_decode(int B, int Hq, int M, int D, int Hk, int capacity_tokens,
 // Workgroups to launch for a plan on the current device (<= plan.wgs), for the
 // decode kernel variant the arguments select.
 int decode_launch_wgs(const DecodePlan& plan, const AttnParams& p, int D);
-// Units a segment start is charged in the paged decode split: the dependent
-// chain that opens a (sequence, KV head) segment, measured in streamed units
-// with two decode workgroups per CU (a sweep of 0-32 peaks at 12-16 for both
-// benchmark decode shapes).
-constexpr int kSegmentCost = 12;
+// Units a segment start is charged in the split of paged and contiguous calls
+// (p.dec_rows set): the dependent chain that opens a (sequence, KV head)
+// segment and the merge that ends it, measured in streamed units. On
+// decode_kernel a sweep of 0-32 peaks at 12-16 for both benchmark decode
+// shapes. decode_wide_kernel's segments cost more (their first tile and Q
+// arrive 5.7 us after the segment begins, its merge takes 2-3 us, and a unit
+// streams in 0.3 us): of 12, 24, 32 and 40, at 24 sequences of 1024-8192 keys
+// and 64/8 heads, M = 5 takes 107, 106, 102 and 100 us, M = 8 111, 113, 108 and
+// 112; 60 sequences, 40/8 heads, M = 7 229, 220, 215 and 214. 0 where rows are
+// loaded one by one.
+int decode_segment_cost(const AttnParams& p);
+
 // Whether paged attention with M query rows per sequence runs on the decode
 // kernels (split over the device, partial results merged by a second
 // kernel; needs the workspace of plan_decode) or on the prefill kernel.

@@ -247,12 +247,11 @@ __device__ __forceinline__ void unit_prefix(const AttnParams& p, int* s_units, i
 }
 
 // Cost split of the unit list. A workgroup that starts a (b, hk) segment
-// pays a dependent chain (key count, head scan, Q, page lookup, first K/V);
-// with two workgroups per CU contending for memory, that takes about as long
-// as streaming kSegmentCost units (p.dec_seg_cost; 0 for the one-per-CU
-// per-row variant). Unit u costs u + P * seg(u), seg(u) = b * Hk + hk being
-// its segment's index (empty segments included), and workgroup w owns the
-// units whose cost lies in [floor(w * C / W), floor((w + 1) * C / W)),
+// pays a dependent chain (key count, head scan, Q, page lookup, first K/V) and a
+// merge at its end, about as long as streaming p.dec_seg_cost units
+// (decode_segment_cost). Unit u costs u + P * seg(u), seg(u) = b * Hk + hk
+// being its segment's index (empty segments included), and workgroup w owns
+// the units whose cost lies in [floor(w * C / W), floor((w + 1) * C / W)),
 // C = U + P * B * Hk. With P = 0 this is the plain equal split of units; P is
 // 0 unless there are at least 2W units, so that every workgroup's cost range
 // holds two or more costs. Measured against the equal split: cfg3 +5 %,
@@ -832,7 +831,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(AttnParams p) {
 //
 // The 16x16 tiles of decode_kernel spend a softmax on 4 keys per lane and a
 // half-rate MFMA on PV; with four 16-row blocks (24 sequences of 1024-8192
-// keys, 64/8 heads, M = 5: 390 MB) they took 121 us against 94 here, with two
+// keys, 64/8 heads, M = 5: 390 MB) they took 121 us against 84 here, with two
 // (M = 3) 96 against 91, and M = 8 157 against 113. Pages of 8 tokens had to
 // load row by row (M = 1: 242 us against 88). One 16-row block of whole-group
 // loads stays on decode_kernel (M = 1: 81 us), whose segments start and merge
@@ -1116,29 +1115,34 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_wide_kernel(AttnParams 
         }
       }
       __syncthreads();
-      for (int e = tid; e < NB * 32 * CF; e += kDecodeThreads) {
-        const int row = e / CF, ch = e % CF;
+      // four rows per thread at a time, without a branch between their LDS
+      // reads (one at a time took 2.4 us of a segment)
+      constexpr int kStep = kDecodeThreads / CF;  // rows per step of the workgroup
+      const int ch = tid % CF;
+#pragma unroll 4
+      for (int row = tid / CF; row < NB * 32; row += kStep) {
         const int ri = rc0 + row;          // row of the slot
-        if (ri >= nrows || ri >= p.dec_rows) break;  // rows past the slot: NaN in the combine
         float mx = s_m[0][row];
 #pragma unroll
         for (int w = 1; w < kDecodeWaves; ++w) mx = fmaxf(mx, s_m[w][row]);
+        const float mz = mx == -INFINITY ? 0.f : mx;  // no visible key: all weights 0
         float lsum = 0.f;
         floatx4 osum = floatx4{0.f, 0.f, 0.f, 0.f};
-        if (mx != -INFINITY) {
 #pragma unroll
-          for (int w = 0; w < kDecodeWaves; ++w) {
-            const float a = __builtin_amdgcn_exp2f(s_m[w][row] - mx);
-            lsum += a * s_l[w][row];
-            osum += a * *reinterpret_cast<const floatx4*>(smem + w * 4 * TILE + row * 4 * D +
-                                                          16 * (ch ^ (row % CF)));
-          }
+        for (int w = 0; w < kDecodeWaves; ++w) {
+          const float a = __builtin_amdgcn_exp2f(s_m[w][row] - mz);
+          lsum += a * s_l[w][row];
+          osum += a * *reinterpret_cast<const floatx4*>(smem + w * 4 * TILE + row * 4 * D +
+                                                        16 * (ch ^ (row % CF)));
         }
-        const int64_t srow = (int64_t)slot * p.dec_rows + ri;
-        *reinterpret_cast<floatx4u*>(p.ws_o + srow * D + 4 * ch) = osum;
-        if (ch == 0) {
-          p.ws_ml[srow * 2 + 0] = mx;
-          p.ws_ml[srow * 2 + 1] = lsum;
+        // rows past the slot: NaN in the combine
+        if (ri < nrows && ri < p.dec_rows) {
+          const int64_t srow = (int64_t)slot * p.dec_rows + ri;
+          *reinterpret_cast<floatx4u*>(p.ws_o + srow * D + 4 * ch) = osum;
+          if (ch == 0) {
+            p.ws_ml[srow * 2 + 0] = mx;
+            p.ws_ml[srow * 2 + 1] = lsum;
+          }
         }
       }
       __syncthreads();  // the stages, s_m and s_l are free again
@@ -1499,6 +1503,11 @@ bool fused_append_ok(int B, int M, int Hq, int Hk, int heads_per_kv, int PS) {
   if (!use_decode_path(B, M, Hq, Hk, heads_per_kv)) return false;
   const int64_t hpk = heads_per_kv <= 0 || heads_per_kv > Hq ? Hq : heads_per_kv;
   return hpk * M <= 2 * kRows && !decode_is_wide(true, PS, (int)(hpk * M));
+}
+
+int decode_segment_cost(const AttnParams& p) {
+  const DecodeVariant v = decode_variant(p);
+  return v.wide_nb > 0 ? 32 : v.aligned ? 12 : 0;
 }
 
 int decode_launch_wgs(const DecodePlan& plan, const AttnParams& p, int D) {
