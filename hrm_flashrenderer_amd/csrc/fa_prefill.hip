@@ -572,8 +572,16 @@ __device__ __forceinline__ void dma_slab(const QuarterSrc& q, const uint32_t* vo
 // -> 90 us; 32/8 heads, D = 64, 512 rows over 8000 keys 127 -> 63 us.
 enum PrefillMode { kWhole, kSplit, kMerge };
 
-template <int D, bool PACKED, int MODE>
-__global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, PrefillGrid g) {
+//
+// GROUPS = 2 (kWhole, per-head tiles): two groups of four waves share the
+// item's rows and take its key tiles alternately, each with its own K/V stages;
+// group 1 hands its state to group 0 through LDS at the end. The item's chain
+// of tiles is half as long, which is what bounds a grid with an item or less
+// per CU (two_groups).
+template <int D, bool PACKED, int MODE, int GROUPS>
+__global__ __launch_bounds__(kThreads * GROUPS, GROUPS == 1 ? 3 : D == 64 ? 2 : 1)
+void prefill_b32_kernel(AttnParams p, PrefillGrid g) {
+  static_assert(GROUPS == 1 || (GROUPS == 2 && MODE == kWhole && !PACKED), "groups: whole items");
   using C = DmaCfg<D>;
   constexpr int BN = 32;
   constexpr int NW = 4;
@@ -589,7 +597,9 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
   // stages: a third gained nothing there.
   constexpr int NST = PACKED ? 3 : 2;
   constexpr int kDmaPerTile = 2 * Slab<D, NW, BN>::IPW;  // DMA instructions per wave and tile
-  __shared__ __attribute__((aligned(1024))) char smem[2 * NST * TILE];  // K0 V0 K1 V1 (K2 V2)
+  // per group K0 V0 K1 V1 (K2 V2)
+  __shared__ __attribute__((aligned(1024))) char smem_all[GROUPS * 2 * NST * TILE];
+  __shared__ float s_state[GROUPS == 2 ? kThreads : 1][2];  // group 1's max and sum per lane
   // PACKED: the q heads of the pair's KV head in head-map order, and the
   // heads whose head-map entry is outside [0, Hk) (collected by the pairs of
   // KV head 0); s_pk_n holds both counts.
@@ -675,7 +685,9 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
   const int hk_pair = pair - b * ngroups;  // PACKED: the pair's KV head
   const int hq = PACKED ? 0 : hk_pair * group + head;
 
-  const int tid = threadIdx.x;
+  const int grp = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / kThreads);
+  const int tid = GROUPS == 1 ? (int)threadIdx.x : (int)threadIdx.x & (kThreads - 1);
+  char* const smem = smem_all + grp * 2 * NST * TILE;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31;
@@ -812,6 +824,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
   const char* kp = reinterpret_cast<const char*>(p.k);
   const char* vp = reinterpret_cast<const char*>(p.v);
   const SlabLane<D, NW, BN> dl = slab_lane<D, NW, BN>(wave, lane);
+  t0 += grp;  // this group's tiles t0, t0 + GROUPS, ...
   QuarterSrc next_src = QuarterSrc{0, 0u};
   if constexpr (MODE != kMerge) {
     if (t0 < ntiles) {
@@ -826,7 +839,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
         dma_slab<D, NW, BN, PACKED>(s1, dl.vv, vp, wave, smem + 3 * TILE);
       }
     }
-    next_src = pages.get(p, b, t0 + NST - 1, kv_len, wave, lane);
+    next_src = pages.get(p, b, t0 + (NST - 1) * GROUPS, kv_len, wave, lane);
 
     if (p.rope_cos != nullptr && q_ok) rope_fragment<KSTEPS, 16>(qreg, p, qo + qrow, 8 * half_id);
   }
@@ -877,12 +890,13 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();
-    if (t + (NST - 1) < ntiles) {
+    if (t + (NST - 1) * GROUPS < ntiles) {
       constexpr int NEXT = (PB + NST - 1) % NST;  // the stage tile t + NST - 1 goes to
       char* nbuf = smem + NEXT * 2 * TILE;
       dma_slab<D, NW, BN, PACKED>(next_src, dl.vk, kp, wave, nbuf);
       dma_slab<D, NW, BN, PACKED>(next_src, dl.vv, vp, wave, nbuf + TILE);
-      if (t + NST < ntiles) next_src = pages.get(p, b, t + NST, kv_len, wave, lane);
+      if (t + NST * GROUPS < ntiles)
+        next_src = pages.get(p, b, t + NST * GROUPS, kv_len, wave, lane);
     }
     if (k0 >= wave_lim_max) return;
     const char* buf = smem + PB * 2 * TILE;
@@ -964,9 +978,12 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
     __builtin_amdgcn_s_setprio(0);
   };
   // (kMerge: t0 = 0 and ntiles are the whole item's; its pieces ran them)
-  for (int t = MODE == kMerge ? ntiles : t0; t < ntiles; t += NST) {
+  // Both groups run the same number of steps (and barriers); a step past the
+  // last tile computes nothing, its keys being past every limit.
+  const int end = GROUPS == 1 ? ntiles : grp + (ntiles + 1) / 2 * 2;
+  for (int t = MODE == kMerge ? end : t0; t < end; t += NST * GROUPS) {
     step(std::integral_constant<int, 0>{}, t);
-    if (t + 1 < ntiles) step(std::integral_constant<int, 1>{}, t + 1);
+    if (t + GROUPS < end) step(std::integral_constant<int, 1>{}, t + GROUPS);
     if constexpr (NST == 3) {
       if (t + 2 < ntiles) step(std::integral_constant<int, 2>{}, t + 2);
     }
@@ -1024,29 +1041,68 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_b32_kernel(AttnParams p, 
       }
     }
   }
+  if constexpr (GROUPS == 2) {
+    // group 1's state, in the lanes' order, over both groups' stages (which
+    // are exactly its size); then group 0 merges it in log2 space
+    static_assert(GROUPS * 2 * NST * TILE == kThreads * 16 * DBLK * 4, "state in the stages");
+    floatx4* st = reinterpret_cast<floatx4*>(smem_all) + tid;
+    __syncthreads();  // every wave has finished reading the last K/V stage
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < DBLK; ++i) {
+#pragma unroll
+        for (int gr = 0; gr < 4; ++gr)
+          st[(4 * i + gr) * kThreads] = floatx4{acc_o[i][4 * gr], acc_o[i][4 * gr + 1],
+                                                acc_o[i][4 * gr + 2], acc_o[i][4 * gr + 3]};
+      }
+      s_state[tid][0] = m_ref;
+      s_state[tid][1] = l_tot;
+    }
+    __syncthreads();
+    if (grp == 0) {
+      const float m1 = s_state[tid][0];
+      const float m_all = fmaxf(m_ref, m1);
+      // a group whose keys the row does not see has the max -inf: weight 0
+      const float w0 = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_all);
+      const float w1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m_all);
+      l_tot = w0 * l_tot + w1 * s_state[tid][1];
+#pragma unroll
+      for (int i = 0; i < DBLK; ++i) {
+#pragma unroll
+        for (int gr = 0; gr < 4; ++gr) {
+          const floatx4 x = st[(4 * i + gr) * kThreads];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc_o[i][4 * gr + r] = w0 * acc_o[i][4 * gr + r] + w1 * x[r];
+        }
+      }
+    }
+  }
   const bool finish = MODE != kSplit || parts == 1;
   const float inv = !head_ok ? __builtin_nanf("") : kv_len == 0 ? 0.f : 1.f / l_tot;
   const bool live = qrow < qlen && row_exists;  // padding rows are zeros whatever their Q held
   __syncthreads();  // every wave has finished reading the last K/V stage
   if (finish) {
     const int lrow = rblk * 32 + col;
+    // (group 0 alone; its own stages hold the 128 rows)
+    if (grp == 0) {
 #pragma unroll
-    for (int i = 0; i < DBLK; ++i) {
+      for (int i = 0; i < DBLK; ++i) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        half4 h = half4{(f16)(acc_o[i][4 * g + 0] * inv), (f16)(acc_o[i][4 * g + 1] * inv),
-                        (f16)(acc_o[i][4 * g + 2] * inv), (f16)(acc_o[i][4 * g + 3] * inv)};
-        if (!live) h = half4{0, 0, 0, 0};
-        const int chunk = (4 * i + g) ^ C::swz_k(lrow);
-        *reinterpret_cast<half4*>(smem + lrow * C::ROWB + 16 * chunk + 8 * half_id) = h;
+        for (int g = 0; g < 4; ++g) {
+          half4 h = half4{(f16)(acc_o[i][4 * g + 0] * inv), (f16)(acc_o[i][4 * g + 1] * inv),
+                          (f16)(acc_o[i][4 * g + 2] * inv), (f16)(acc_o[i][4 * g + 3] * inv)};
+          if (!live) h = half4{0, 0, 0, 0};
+          const int chunk = (4 * i + g) ^ C::swz_k(lrow);
+          *reinterpret_cast<half4*>(smem + lrow * C::ROWB + 16 * chunk + 8 * half_id) = h;
+        }
       }
     }
     __syncthreads();
     const int rows = min(kBM, (PACKED ? pk_rows : p.M) - q0);
     f16* ob = op + (int64_t)q0 * D;
-    for (int e = tid; e < rows * C::CH; e += kThreads) {
+    for (int e = (int)threadIdx.x; e < rows * C::CH; e += kThreads * GROUPS) {
       const int r = e / C::CH, ch = e % C::CH;
-      const half8 v = *reinterpret_cast<const half8*>(smem + r * C::ROWB + 16 * (ch ^ C::swz_k(r)));
+      const half8 v = *reinterpret_cast<const half8*>(smem_all + r * C::ROWB + 16 * (ch ^ C::swz_k(r)));
       f16* dst;
       if constexpr (PACKED) {
         const int pr = q0 + r, j = pr / p.M;
@@ -1563,6 +1619,14 @@ static PrefillPlan plan_prefill(const AttnParams& p, int D) {
   return plan;
 }
 
+// Whether two wave groups per item serve a whole-item grid better than one:
+// with an item or less per CU the second group takes idle wave slots. 8 heads,
+// D = 128, 2 x 1400 rows (176 items) 31.5 -> 25.6 us; 32 heads x 1024 rows (256
+// items) 24.5 -> 21.7 us, D = 64 19.1 -> 16.4 us. Beyond that the groups share
+// a CU with other items and the merge is paid for nothing: D = 64, 1024 items
+// of 512-row heads 21 us with one group, 25 us with two.
+static bool two_groups(const PrefillGrid& g) { return g.slots <= 256; }
+
 template <int D, bool PACKED>
 static hipError_t launch_b32(AttnParams p, const PrefillPlan& plan, hipStream_t stream) {
   const dim3 slots((unsigned)plan.g.slots), block(kThreads);
@@ -1570,10 +1634,17 @@ static hipError_t launch_b32(AttnParams p, const PrefillPlan& plan, hipStream_t 
     p.ws_o = reinterpret_cast<float*>(p.ws);
     p.ws_ml = reinterpret_cast<float*>(reinterpret_cast<char*>(p.ws) + plan.o_bytes);
     const dim3 all((unsigned)(plan.g.slots * plan.g.pieces));
-    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kSplit>), all, block, 0, stream, p, plan.g);
-    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kMerge>), slots, block, 0, stream, p, plan.g);
+    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kSplit, 1>), all, block, 0, stream, p, plan.g);
+    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kMerge, 1>), slots, block, 0, stream, p, plan.g);
   } else {
-    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kWhole>), slots, block, 0, stream, p, plan.g);
+    if constexpr (!PACKED) {
+      if (two_groups(plan.g)) {
+        hipLaunchKernelGGL((prefill_b32_kernel<D, false, kWhole, 2>), slots, dim3(2 * kThreads), 0,
+                           stream, p, plan.g);
+        return hipGetLastError();
+      }
+    }
+    hipLaunchKernelGGL((prefill_b32_kernel<D, PACKED, kWhole, 1>), slots, block, 0, stream, p, plan.g);
   }
   return hipGetLastError();
 }

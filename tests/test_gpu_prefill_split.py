@@ -70,3 +70,20 @@ def test_split_in_a_graph(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, flash_attn(q, k, v, True, 2244))
+
+
+@pytest.mark.parametrize("Hq,Hk,M,N,D,causal", [
+    (8, 8, 129, 129, 128, True),    # two items per head, the second with one live row
+    (4, 2, 300, 31, 64, False),     # one key tile: group 1 has none
+    (6, 3, 200, 1000, 128, True),   # rows that do not see group 1's last tile
+    (32, 8, 1024, 1024, 64, True),  # 256 items: the largest such grid
+    (33, 3, 1024, 1024, 64, True),  # 264 items: one group
+])
+def test_two_groups(gpu, Hq, Hk, M, N, D, causal):
+    """Grids of at most 256 items run two wave groups per item."""
+    q, k, v = seeded((1, Hq, M, D), 1), seeded((1, Hk, N, D), 2), seeded((1, Hk, N, D), 3)
+    out = flash_attn(q, k, v, causal, max(0, N - M))
+    for h in (0, Hq // 2, Hq - 1):
+        ref = ora.attention_f64(q[:, h:h + 1].cpu(), k[:, h * Hk // Hq:h * Hk // Hq + 1].cpu(),
+                                v[:, h * Hk // Hq:h * Hk // Hq + 1].cpu(), causal, max(0, N - M), 0)
+        assert_close(out[:, h:h + 1].cpu().numpy(), ref, f"h={h}")
