@@ -235,8 +235,8 @@ static int contig_fwd(const void* q, const void* k, const void* v, void* o, int 
       pc.ws_units = reinterpret_cast<int*>(ws + plan.o_bytes + plan.ml_bytes);
       pc.ws_app = pc.ws_units + (Bc + 1);
       pc.dec_rows = cplan.rows;
-      pc.dec_seg_cost = fa::decode_segment_cost(pc);
       pc.dec_wgs = fa::decode_launch_wgs(cplan, pc, D);
+      pc.dec_seg_cost = fa::decode_segment_cost(pc);
       e = fa::launch_decode(pc, D, (hipStream_t)stream);
     }
     return launch_status(e);
@@ -403,8 +403,8 @@ static int paged_fwd(const void* q, const void* k_pages, const void* v_pages,
       pc.ws_app = pc.ws_units + (Bc + 1);
       // every field decode_variant reads is set before the occupancy query
       pc.dec_rows = cplan.rows;
-      pc.dec_seg_cost = fa::decode_segment_cost(pc);
       pc.dec_wgs = fa::decode_launch_wgs(cplan, pc, D);
+      pc.dec_seg_cost = fa::decode_segment_cost(pc);
       e = fa::launch_decode(pc, D, (hipStream_t)stream);
     }
     combine_advances = true;

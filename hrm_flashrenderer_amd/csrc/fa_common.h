@@ -309,7 +309,7 @@ DecodePlan plan_decode(int B, int Hq, int M, int D, int Hk, int capacity_tokens,
 // decode kernel variant the arguments select.
 int decode_launch_wgs(const DecodePlan& plan, const AttnParams& p, int D);
 // Units a segment start is charged in the split of paged and contiguous calls
-// (p.dec_rows set): the dependent chain that opens a (sequence, KV head)
+// (p.dec_rows and p.dec_wgs set): the dependent chain that opens a (sequence, KV head)
 // segment and the merge that ends it, measured in streamed units. On
 // decode_kernel a sweep of 0-32 peaks at 12-16 for both benchmark decode
 // shapes. decode_wide_kernel's segments cost more (their first tile and Q
