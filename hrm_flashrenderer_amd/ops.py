@@ -12,8 +12,9 @@ conventions as the reference, flashattention_custom/ops.py:79-99):
 Each validates its arguments in Python with the reference extension's
 messages (csrc/ext.cpp:30-89), then calls a `torch.library` custom op
 (`hrm_fa::*`), or for plain tensors its body at once (`_direct`), which calls
-the C ABI of libfa_mi355x.so on the current stream of the tensors' device. There is no CPU fallback: tensors must be on a
-ROCm device and the library must be built, otherwise a RuntimeError is raised
+the C ABI of libfa_mi355x.so on the current stream of the tensors' device.
+There is no CPU fallback: tensors must be on a ROCm device and the library must
+be built, otherwise a RuntimeError is raised
 (the reference's `_ext` raises the same "CUDA required" checks; the wording
 refers to torch's device type, which is "cuda" on ROCm).
 
@@ -221,8 +222,8 @@ def _prefill_split_bytes(B: int, Hq: int, Hk: int, M: int, D: int, keys: int, hp
 # --------------------------------------------------------------------------
 
 def _flash_attn_body(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool,
-                   q_offset: int, k_offset: int, q_offsets: Optional[torch.Tensor],
-                   k_offsets: Optional[torch.Tensor]) -> torch.Tensor:
+                     q_offset: int, k_offset: int, q_offsets: Optional[torch.Tensor],
+                     k_offsets: Optional[torch.Tensor]) -> torch.Tensor:
     lib = _lib.load()
     o = torch.empty_like(q)
     B, Hq, M, D = q.shape
@@ -251,13 +252,13 @@ def _(q, k, v, causal, q_offset, k_offset, q_offsets, k_offsets):
 
 
 def _flash_attn_paged_body(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
-                         seqlen: torch.Tensor, page_size: int, head_map: torch.Tensor,
-                         causal: bool, q_offset: int, k_offset: int,
-                         q_offsets: Optional[torch.Tensor], k_offsets: Optional[torch.Tensor],
-                         block_table: Optional[torch.Tensor], rope_cos: Optional[torch.Tensor],
-                         rope_sin: Optional[torch.Tensor],
-                         q_lens: Optional[torch.Tensor] = None,
-                         heads_per_kv: int = 0) -> torch.Tensor:
+                           seqlen: torch.Tensor, page_size: int, head_map: torch.Tensor,
+                           causal: bool, q_offset: int, k_offset: int,
+                           q_offsets: Optional[torch.Tensor], k_offsets: Optional[torch.Tensor],
+                           block_table: Optional[torch.Tensor], rope_cos: Optional[torch.Tensor],
+                           rope_sin: Optional[torch.Tensor],
+                           q_lens: Optional[torch.Tensor] = None,
+                           heads_per_kv: int = 0) -> torch.Tensor:
     lib = _lib.load()
     o = torch.empty_like(q)
     B, Hq, M, D = q.shape
@@ -281,7 +282,8 @@ def _flash_attn_paged_body(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torc
     return o
 
 
-_flash_attn_paged_op = torch.library.custom_op("hrm_fa::flash_attn_paged", mutates_args=())(_flash_attn_paged_body)
+_flash_attn_paged_op = torch.library.custom_op(
+    "hrm_fa::flash_attn_paged", mutates_args=())(_flash_attn_paged_body)
 
 
 @_flash_attn_paged_op.register_fake
@@ -291,9 +293,9 @@ def _(q, k_pages, v_pages, seqlen, page_size, head_map, causal, q_offset, k_offs
 
 
 def _paged_kv_append_body(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: torch.Tensor,
-                        v_new: torch.Tensor, start_pos: int, start_positions: Optional[torch.Tensor],
-                        page_size: int, block_table: Optional[torch.Tensor],
-                        rope_cos: Optional[torch.Tensor], rope_sin: Optional[torch.Tensor]) -> None:
+                          v_new: torch.Tensor, start_pos: int, start_positions: Optional[torch.Tensor],
+                          page_size: int, block_table: Optional[torch.Tensor],
+                          rope_cos: Optional[torch.Tensor], rope_sin: Optional[torch.Tensor]) -> None:
     lib = _lib.load()
     B, Hk, T, D = k_new.shape
     NB, P = k_pages.size(0), k_pages.size(2)
@@ -309,7 +311,8 @@ def _paged_kv_append_body(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: t
                 *args, rope_cos.data_ptr(), rope_sin.data_ptr(), rope_cos.size(0), stream))
 
 
-_paged_kv_append_op = torch.library.custom_op("hrm_fa::paged_kv_append", mutates_args=("k_pages", "v_pages"))(_paged_kv_append_body)
+_paged_kv_append_op = torch.library.custom_op(
+    "hrm_fa::paged_kv_append", mutates_args=("k_pages", "v_pages"))(_paged_kv_append_body)
 
 
 @_paged_kv_append_op.register_fake
@@ -319,13 +322,13 @@ def _(k_pages, v_pages, k_new, v_new, start_pos, start_positions, page_size, blo
 
 
 def _flash_attn_paged_append_body(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
-                                seqlen: torch.Tensor, page_size: int, head_map: torch.Tensor,
-                                causal: bool, q_offset: int, q_offsets: Optional[torch.Tensor],
-                                block_table: Optional[torch.Tensor], k_new: torch.Tensor,
-                                v_new: torch.Tensor, advance: bool, start_pos: int,
-                                start_positions: Optional[torch.Tensor],
-                                rope_cos: Optional[torch.Tensor], rope_sin: Optional[torch.Tensor],
-                                heads_per_kv: int = 0) -> torch.Tensor:
+                                  seqlen: torch.Tensor, page_size: int, head_map: torch.Tensor,
+                                  causal: bool, q_offset: int, q_offsets: Optional[torch.Tensor],
+                                  block_table: Optional[torch.Tensor], k_new: torch.Tensor,
+                                  v_new: torch.Tensor, advance: bool, start_pos: int,
+                                  start_positions: Optional[torch.Tensor],
+                                  rope_cos: Optional[torch.Tensor], rope_sin: Optional[torch.Tensor],
+                                  heads_per_kv: int = 0) -> torch.Tensor:
     lib = _lib.load()
     o = torch.empty_like(q)
     B, Hq, M, D = q.shape
@@ -347,7 +350,8 @@ def _flash_attn_paged_append_body(q: torch.Tensor, k_pages: torch.Tensor, v_page
     return o
 
 
-_flash_attn_paged_append_op = torch.library.custom_op("hrm_fa::flash_attn_paged_append", mutates_args=("k_pages", "v_pages", "seqlen"))(_flash_attn_paged_append_body)
+_flash_attn_paged_append_op = torch.library.custom_op(
+    "hrm_fa::flash_attn_paged_append", mutates_args=("k_pages", "v_pages", "seqlen"))(_flash_attn_paged_append_body)
 
 
 @_flash_attn_paged_append_op.register_fake
@@ -357,9 +361,9 @@ def _(q, k_pages, v_pages, seqlen, page_size, head_map, causal, q_offset, q_offs
 
 
 def _paged_kv_scatter_body(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: torch.Tensor,
-                         v_new: torch.Tensor, positions: torch.Tensor, page_size: int,
-                         block_table: Optional[torch.Tensor], rope_cos: Optional[torch.Tensor],
-                         rope_sin: Optional[torch.Tensor]) -> None:
+                           v_new: torch.Tensor, positions: torch.Tensor, page_size: int,
+                           block_table: Optional[torch.Tensor], rope_cos: Optional[torch.Tensor],
+                           rope_sin: Optional[torch.Tensor]) -> None:
     lib = _lib.load()
     B, Hk, T, D = k_new.shape
     NB, P = k_pages.size(0), k_pages.size(2)
@@ -372,7 +376,8 @@ def _paged_kv_scatter_body(k_pages: torch.Tensor, v_pages: torch.Tensor, k_new: 
             stream))
 
 
-_paged_kv_scatter_op = torch.library.custom_op("hrm_fa::paged_kv_scatter", mutates_args=("k_pages", "v_pages"))(_paged_kv_scatter_body)
+_paged_kv_scatter_op = torch.library.custom_op(
+    "hrm_fa::paged_kv_scatter", mutates_args=("k_pages", "v_pages"))(_paged_kv_scatter_body)
 
 
 @_paged_kv_scatter_op.register_fake
